@@ -410,7 +410,19 @@ def _add(a, b):
     return binop("add", a, b)
 
 
+def _is_factor(e):
+    """A finite nonzero constant."""
+    return e.op == "const" and e.dtype != "b" and e.value != 0 and math.isfinite(float(e.value))
+
+
 def _mul(a, b):
+    # constant factors collect into one: the derivative of c tanh(s / c) is 1 - tanh^2
+    if _is_factor(a) and not _is_factor(b):
+        a, b = b, a
+    if _is_factor(b) and a.op == "mul" and a.dtype == "f":
+        for x, k in (a.args, a.args[::-1]):
+            if _is_factor(k) and math.isfinite(float(k.value) * float(b.value)):
+                return _mul(x, _fconst(float(k.value) * float(b.value)))
     if _is(a, 0.0) or _is(b, 0.0) or _is(a, 0) or _is(b, 0):
         return ZERO
     if _is(a, 1.0):
@@ -438,6 +450,9 @@ def derivative(e: Expr) -> Expr:
         return _add(_mul(derivative(a[0]), a[1]), _mul(a[0], derivative(a[1])))
     if op == "truediv":
         da, db = derivative(a[0]), derivative(a[1])
+        if _is(db, 0.0) or _is(db, 0):  # constant divisor: (u / c)' = u' (1 / c)
+            inv = _fconst(1.0 / float(np.float32(a[1].value))) if _is_factor(a[1]) else binop("truediv", ONE, a[1])
+        return _mul(da, inv)
         num = _add(_mul(da, a[1]), _mul(_fconst(-1), _mul(a[0], db)))
         return binop("truediv", num, binop("mul", a[1], a[1])) if not _is(num, 0.0) else ZERO
     if op == "neg":
@@ -485,8 +500,32 @@ def derivative(e: Expr) -> Expr:
 # -------------------------------------------------------------- codegen ----
 _CTYPE = {"i": "int", "f": "float", "b": "bool"}
 _CBIN = {"add": "+", "sub": "-", "mul": "*", "lt": "<", "le": "<=", "gt": ">", "ge": ">=", "eq": "==", "ne": "!="}
-_CFUN = {"tanh": "tanhf", "exp": "expf", "log": "logf", "sqrt": "sqrtf", "exp2": "exp2f", "log2": "log2f",
+_CFUN = {"tanh": "um_tanh", "exp": "expf", "log": "logf", "sqrt": "sqrtf", "exp2": "exp2f", "log2": "log2f",
          "sin": "sinf", "cos": "cosf", "floor": "floorf", "ceil": "ceilf"}
+
+
+# evaluated once where the score and its derivative share them (the compiler's
+# own elimination gave up on the unrolled tiles: three tanh per score)
+_HOISTED = set(_CFUN) | {"sigmoid", "pow", "truediv"}
+
+
+def _shared(roots) -> List[Expr]:
+    """Nodes of `roots` with a function or division that occurs more than
+    once, innermost first."""
+    seen: Dict[str, int] = {}
+    order: List[Expr] = []
+
+    def walk(e):
+        for x in e.args:
+            walk(x)
+        if e.op in _HOISTED and "score" in e.uses():
+            code = emit(e)
+            seen[code] = seen.get(code, 0) + 1
+            if seen[code] == 1:
+                order.append(e)
+    for r in roots:
+        walk(r)
+    return [e for e in order if seen[emit(e)] > 1]
 
 
 def _cast(code: str, src: str, dst: str) -> str:
@@ -495,8 +534,32 @@ def _cast(code: str, src: str, dst: str) -> str:
     return f"(({_CTYPE[dst]})({code}))"
 
 
-def emit(e: Expr) -> str:
-    """C++ expression for e (variables b, h, q, kv, s; tensors through p.mod_buf)."""
+def _reciprocal(e: Expr):
+    """(hi, lo) float literals with hi + lo = 1 / c for a constant divisor c
+    (lo None where hi is exact), or None for a divisor that is no constant or
+    whose parts leave the normal range.  hi is rounded towards zero, so lo has
+    its sign: an infinite dividend stays infinite in x hi + x lo."""
+    if e.op != "const" or e.dtype == "b":
+        return None
+    c = float(np.float32(e.value))
+    if not 2.0 ** -90 < abs(c) < 2.0 ** 90:
+        return None
+    hi = np.float32(1.0 / c)
+    if abs(float(hi)) > abs(1.0 / c):
+        hi = np.nextafter(hi, np.float32(0))
+    lo = np.float32(1.0 / c - float(hi))
+    text = [f"({v.hex()}f)" for v in (float(hi), float(lo))]
+    return text[0], (None if lo == 0 else text[1])
+
+
+def emit(e: Expr, names: Optional[Dict[str, str]] = None) -> str:
+    """C++ expression for e (variables b, h, q, kv, s; tensors through
+    p.mod_buf); `names`: the locals that hold subexpressions, by their code."""
+    if names and e.op in _HOISTED and emit(e) in names:
+        return names[emit(e)]
+
+    def em(x):
+        return emit(x, names)
     op, a = e.op, e.args
     if op == "const":
         if e.dtype == "b":
@@ -516,57 +579,60 @@ def emit(e: Expr) -> str:
         dt = "f" if "f" in (a[0].dtype, a[1].dtype) and op in ("add", "sub", "mul") else None
         if op in ("add", "sub", "mul"):
             t = e.dtype
-            return f"({_cast(emit(a[0]), a[0].dtype, t)} {_CBIN[op]} {_cast(emit(a[1]), a[1].dtype, t)})"
+            return f"({_cast(em(a[0]), a[0].dtype, t)} {_CBIN[op]} {_cast(em(a[1]), a[1].dtype, t)})"
         t = "f" if "f" in (a[0].dtype, a[1].dtype) else "i"
-        return f"({_cast(emit(a[0]), a[0].dtype, t)} {_CBIN[op]} {_cast(emit(a[1]), a[1].dtype, t)})"
+        return f"({_cast(em(a[0]), a[0].dtype, t)} {_CBIN[op]} {_cast(em(a[1]), a[1].dtype, t)})"
     if op == "truediv":
-        return f"({_cast(emit(a[0]), a[0].dtype, 'f')} / {_cast(emit(a[1]), a[1].dtype, 'f')})"
+        x, r = _cast(em(a[0]), a[0].dtype, "f"), _reciprocal(a[1]) if a[0].op != "const" else None
+        if r is not None:
+            return f"({x} * {r[0]})" if r[1] is None else f"um_mul2({x}, {r[0]}, {r[1]})"
+        return f"({x} / {_cast(em(a[1]), a[1].dtype, 'f')})"
     if op in ("floordiv", "mod"):
         if e.dtype == "f":
-            x, y = _cast(emit(a[0]), a[0].dtype, "f"), _cast(emit(a[1]), a[1].dtype, "f")
+            x, y = _cast(em(a[0]), a[0].dtype, "f"), _cast(em(a[1]), a[1].dtype, "f")
             return f"um_f{op}({x}, {y})"
-        return f"um_i{op}({emit(a[0])}, {emit(a[1])})"
+        return f"um_i{op}({em(a[0])}, {em(a[1])})"
     if op == "pow":
-        x, y = _cast(emit(a[0]), a[0].dtype, "f"), _cast(emit(a[1]), a[1].dtype, "f")
+        x, y = _cast(em(a[0]), a[0].dtype, "f"), _cast(em(a[1]), a[1].dtype, "f")
         if a[1].op == "const" and a[1].value == 2:
             return f"um_sq({x})"
         return f"powf({x}, {y})"
     if op in ("min", "max"):
         if e.dtype == "f":
-            return f"f{op}f({_cast(emit(a[0]), a[0].dtype, 'f')}, {_cast(emit(a[1]), a[1].dtype, 'f')})"
-        return f"{op}({_cast(emit(a[0]), a[0].dtype, 'i')}, {_cast(emit(a[1]), a[1].dtype, 'i')})"
+            return f"f{op}f({_cast(em(a[0]), a[0].dtype, 'f')}, {_cast(em(a[1]), a[1].dtype, 'f')})"
+        return f"{op}({_cast(em(a[0]), a[0].dtype, 'i')}, {_cast(em(a[1]), a[1].dtype, 'i')})"
     if op in ("and", "or", "xor"):
         if e.dtype == "b":
             c = {"and": "&&", "or": "||", "xor": "!="}[op]
         else:
             c = {"and": "&", "or": "|", "xor": "^"}[op]
-        return f"({emit(a[0])} {c} {emit(a[1])})"
+        return f"({em(a[0])} {c} {em(a[1])})"
     if op == "not":
-        return f"(!{emit(a[0])})"
+        return f"(!{em(a[0])})"
     if op == "bitnot":
-        return f"(~{_cast(emit(a[0]), a[0].dtype, 'i')})"
+        return f"(~{_cast(em(a[0]), a[0].dtype, 'i')})"
     if op == "neg":
-        return f"(-{_cast(emit(a[0]), a[0].dtype, e.dtype)})"
+        return f"(-{_cast(em(a[0]), a[0].dtype, e.dtype)})"
     if op == "abs":
-        return f"fabsf({emit(a[0])})" if e.dtype == "f" else f"abs({_cast(emit(a[0]), a[0].dtype, 'i')})"
+        return f"fabsf({em(a[0])})" if e.dtype == "f" else f"abs({_cast(em(a[0]), a[0].dtype, 'i')})"
     if op in _CFUN:
-        return f"{_CFUN[op]}({_cast(emit(a[0]), a[0].dtype, 'f')})"
+        return f"{_CFUN[op]}({_cast(em(a[0]), a[0].dtype, 'f')})"
     if op == "sigmoid":
-        return f"um_sigmoid({_cast(emit(a[0]), a[0].dtype, 'f')})"
+        return f"um_sigmoid({_cast(em(a[0]), a[0].dtype, 'f')})"
     if op == "float":
-        return _cast(emit(a[0]), a[0].dtype, "f")
+        return _cast(em(a[0]), a[0].dtype, "f")
     if op == "int":
-        return _cast(emit(a[0]), a[0].dtype, "i")
+        return _cast(em(a[0]), a[0].dtype, "i")
     if op == "where":
         t = e.dtype
-        return (f"({emit(a[0])} ? {_cast(emit(a[1]), a[1].dtype, t)} : "
-                f"{_cast(emit(a[2]), a[2].dtype, t)})")
+        return (f"({em(a[0])} ? {_cast(em(a[1]), a[1].dtype, t)} : "
+                f"{_cast(em(a[2]), a[2].dtype, t)})")
     if op == "gather":
         slot, shape = e.value
         off, stride = [], 1
         terms = []
         for i in reversed(range(len(shape))):
-            idx = f"um_clamp({_cast(emit(a[i]), a[i].dtype, 'i')}, {shape[i]})"
+            idx = f"um_clamp({_cast(em(a[i]), a[i].dtype, 'i')}, {shape[i]})"
             terms.append(f"(long)({idx}) * {stride}L" if stride != 1 else f"(long)({idx})")
             stride *= shape[i]
         ty = {"f": "float", "i": "int", "b": "int"}[e.dtype]
@@ -590,6 +656,25 @@ __device__ __forceinline__ int um_imod(int a, int b) {
 __device__ __forceinline__ float um_ffloordiv(float a, float b) { return floorf(a / b); }
 __device__ __forceinline__ float um_fmod(float a, float b) { return a - b * floorf(a / b); }
 __device__ __forceinline__ float um_sq(float x) { return x * x; }
+// x times a reciprocal held in two parts (a division by a constant to within
+// 2^-23 of the correctly rounded one, in two instructions instead of the ten
+// of an IEEE division)
+__device__ __forceinline__ float um_mul2(float x, float hi, float lo) { return fmaf(x, hi, x * lo); }
+// tanh without branches.  The math library's tanhf is a divergent branch over
+// two long paths, evaluated per score: the forward and backward of a tanh cap
+// through it took 819 us at B4 H16 S2048 D64 (prefix mask), 422 with this
+// one (366 with the built-in soft-cap).  |x| >= 0.5: 1 - 2 / (2^(2 |x| log2 e) + 1) on the
+// exponential and reciprocal units; below, where that cancels, an odd
+// polynomial (minimax in x^2, 2^-26 relative).  Within 4 * 2^-24 relative.
+__device__ __forceinline__ float um_tanh(float x) {
+  const float a = fabsf(x), y = x * x;
+  const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a * 2.8853900817779268f) + 1.0f);
+  const float big = fmaf(-2.0f, r, 1.0f);
+  float p = fmaf(0.01725698875064151f, y, -0.05305294934872954f);
+  p = fmaf(p, y, 0.13325987273043643f);
+  p = fmaf(p, y, -0.33333148377139477f);
+  return a < 0.5f ? fmaf(x * y, p, x) : copysignf(big, x);
+}
 __device__ __forceinline__ float um_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 }  // namespace um
 """
@@ -609,8 +694,12 @@ def policy_source(mask: Optional[Expr], score: Optional[Expr]) -> str:
              "    using namespace um;"]
     if score is not None:
         d = derivative(score)
-        lines += [f"    *dsds = {_cast(emit(d), d.dtype, 'f')};",
-                  f"    return {_cast(emit(score), score.dtype, 'f')};"]
+        names: Dict[str, str] = {}
+        for i, e in enumerate(_shared([score, d])):
+            lines.append(f"    const float t{i} = {emit(e, names)};")
+            names[emit(e)] = f"t{i}"
+        lines += [f"    *dsds = {_cast(emit(d, names), d.dtype, 'f')};",
+                  f"    return {_cast(emit(score, names), score.dtype, 'f')};"]
     else:
         lines += ["    *dsds = 1.0f;", "    return s;"]
     lines += ["  }", "};", ""]

@@ -200,3 +200,27 @@ def test_builtin_score_params_need_a_blob_built_for_them():
         torch.cuda.synchronize()
     finally:
         _lib.check(lib.fa_mods_unload(h))
+
+
+@pytest.mark.parametrize("name", ["tanh", "tanh-small-scale", "divide-by-constant"])
+def test_generated_functions_to_float32_rounding(name):
+    """With a single key the LSE is the score itself, so the generated tanh (polynomial below 0.5,
+    exponential above) and the division by a constant are read off directly: every value within
+    8 * 2^-24 of float64 (4 of the function, 2 roundings of the log2 conversions, the input's scaling)."""
+    import torch
+    pf = _pf()
+    x = np.concatenate([np.geomspace(1e-6, 30.0, 2000), [0.49999997, 0.5, 0.50000006]]).astype(np.float32)
+    x = np.concatenate([x, -x])
+    score, want = {
+        "tanh": (lambda s, b, h, q, kv: torch.tanh(s), np.tanh(x.astype(np.float64))),
+        "tanh-small-scale": (lambda s, b, h, q, kv: 1024.0 * torch.tanh(s / 1024.0),
+                             1024.0 * np.tanh(x.astype(np.float64) / 1024.0)),
+        "divide-by-constant": (lambda s, b, h, q, kv: s / 3.7, x.astype(np.float64) / np.float64(np.float32(3.7))),
+    }[name]
+    q = torch.zeros(1, 1, x.size, 32, device="cuda")
+    q[0, 0, :, 0] = torch.from_numpy(x).cuda()
+    k = torch.zeros(1, 1, 1, 32, device="cuda")
+    k[..., 0] = 1.0
+    _, lse = pf.flex_attention(q, k, torch.ones_like(k), score_mod=score, scale=1.0, return_lse=True)
+    got = lse[0, 0].double().cpu().numpy()
+    assert np.max(np.abs(got - want) / np.abs(want)) <= 8 * 2.0 ** -24

@@ -178,3 +178,14 @@ def test_blob_from_other_kernel_headers_is_refused():
     assert load(bad) == FA_ERR_SHAPE
     assert load(blob[:-1]) == FA_ERR_SHAPE  # truncated code object
     assert load(blob[:20]) == FA_ERR_SHAPE  # shorter than the header
+
+
+def test_shared_functions_and_constant_factors_are_emitted_once():
+    """A soft-cap's tanh serves the score and its derivative, whose constant factors cancel."""
+    low = L.lower_score(lambda s, b, h, q, kv: 30.0 * torch.tanh(s / 30.0))
+    src = L.policy_source(None, low.expr)
+    body = src[src.index("struct UserMod"):]
+    assert body.count("um_tanh(") == 1 and " / " not in body
+    assert "*dsds = ((1.0f) - (t1 * t1));" in body
+    # a divisor without a reciprocal in the normal range keeps its division
+    assert "/ (0.0f)" in L.policy_source(None, L.lower_score(lambda s, b, h, q, kv: s / 0.0).expr)
