@@ -42,7 +42,7 @@ FLAGS = [
 
 
 # kernel headers the library embeds for run-time compiles of user mods
-RTC_HEADERS = ["index.h", "common.h", "dma.h", "kargs.h", "fwd.h", "fwd_bf16.h", "bwd.h", "bwd_bf16.h"]
+RTC_HEADERS = ["index.h", "common.h", "dma.h", "kargs.h", "fwd.h", "fwd_bf16.h", "bwd.h", "bwd_bf16.h", "f32_split.h"]
 GEN_DIR = os.path.join(HERE, "_build")
 
 

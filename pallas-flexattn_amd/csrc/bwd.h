@@ -75,8 +75,13 @@ __global__ __launch_bounds__(256) void delta_kernel(BwdArgs a, int nrows) {
 using QWalk = QWalkT<DeviceLoad>;
 
 // ----------------------------------------------------------------- dK dV ---
-template <typename T, int D, int BQ, int NW, bool kMods, class Mod = BuiltinMod>
-__global__ __launch_bounds__(NW * 64) void dkdv_kernel(BwdArgs a) {
+// One work item of the general dK/dV; `lds`: dkdv_item_lds() bytes.
+template <typename T, int D, int BQ>
+constexpr int dkdv_item_lds() {
+  return 4 * BQ * D * (int)sizeof(T) + 2 * BQ * 4;
+}
+template <typename T, int D, int BQ, int NW, bool kMods, class Mod>
+__device__ __forceinline__ void dkdv_item(const BwdArgs& a, char* lds) {
   using E = Elt<T>;
   using frag = typename E::frag;
   constexpr int BKV = 32 * NW;
@@ -93,12 +98,12 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(BwdArgs a) {
   using TTile = LdsTile<T, D, BQ, 1>;  // Q^T / dO^T
   static_assert(D % 32 == 0 && BQ % 32 == 0, "tile shape");
 
-  __shared__ __attribute__((aligned(16))) char lds_q[RTile::kBytes];
-  __shared__ __attribute__((aligned(16))) char lds_do[RTile::kBytes];
-  __shared__ __attribute__((aligned(16))) char lds_qt[TTile::kBytes];
-  __shared__ __attribute__((aligned(16))) char lds_dot[TTile::kBytes];
-  __shared__ __attribute__((aligned(16))) float lds_lse[BQ];
-  __shared__ __attribute__((aligned(16))) float lds_dl[BQ];
+  char* const lds_q = lds;
+  char* const lds_do = lds_q + RTile::kBytes;
+  char* const lds_qt = lds_do + RTile::kBytes;
+  char* const lds_dot = lds_qt + TTile::kBytes;
+  float* const lds_lse = reinterpret_cast<float*>(lds_dot + TTile::kBytes);
+  float* const lds_dl = lds_lse + BQ;
 
   const Problem& P = a.p;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -289,9 +294,20 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(BwdArgs a) {
   }
 }
 
+template <typename T, int D, int BQ, int NW, bool kMods, class Mod = BuiltinMod>
+__global__ __launch_bounds__(NW * 64) void dkdv_kernel(BwdArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[dkdv_item_lds<T, D, BQ>()];
+  dkdv_item<T, D, BQ, NW, kMods, Mod>(a, lds);
+}
+
 // -------------------------------------------------------------------- dQ ---
-template <typename T, int D, int BN, int NW, bool kMods, class Mod = BuiltinMod>
-__global__ __launch_bounds__(NW * 64) void dq_kernel(BwdArgs a) {
+// One work item of the general dQ; `lds`: dq_item_lds() bytes.
+template <typename T, int D, int BN>
+constexpr int dq_item_lds() {
+  return 3 * BN * D * (int)sizeof(T);
+}
+template <typename T, int D, int BN, int NW, bool kMods, class Mod>
+__device__ __forceinline__ void dq_item(const BwdArgs& a, char* lds) {
   using E = Elt<T>;
   using frag = typename E::frag;
   constexpr int BM = 32 * NW;
@@ -308,9 +324,9 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(BwdArgs a) {
   using TTile = LdsTile<T, D, BN, 1>;  // K^T
   static_assert(D % 32 == 0 && BN % 32 == 0, "tile shape");
 
-  __shared__ __attribute__((aligned(16))) char lds_k[RTile::kBytes];
-  __shared__ __attribute__((aligned(16))) char lds_v[RTile::kBytes];
-  __shared__ __attribute__((aligned(16))) char lds_kt[TTile::kBytes];
+  char* const lds_k = lds;
+  char* const lds_v = lds_k + RTile::kBytes;
+  char* const lds_kt = lds_v + RTile::kBytes;
 
   const Problem& P = a.p;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -344,27 +360,7 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(BwdArgs a) {
   const float slope = P.alibi ? P.alibi[h] : 0.f;
   const int qdoc = (P.q_doc && qvalid) ? P.q_doc[(size_t)b * P.Sq + qw] : 0;
 
-  KvWalk walk;
-  walk.bn = BN;
-  walk.mblk = P.mblk_kv;
-  walk.sub = P.mblk_kv / BN;
-  walk.nblk = P.n_kvblk;
-  walk.dense = !P.has_tables;
-  walk.ntiles_dense = (P.Skv + BN - 1) / BN;
-  walk.dense_masked = P.has_mask;
-  walk.full = walk.part = nullptr;
-  walk.nfull = walk.npart = 0;
-  if (P.has_tables) {
-    const int row = tab_row(P, b, h, q0 / P.mblk_q, P.n_qblk);
-    if (P.full_kv_num) {
-      walk.nfull = clamp_count(scalar_load(P.full_kv_num, row), P.kv_width);
-      walk.full = P.full_kv_idx + (size_t)row * P.kv_width;
-    }
-    if (P.kv_num) {
-      walk.npart = clamp_count(scalar_load(P.kv_num, row), P.kv_width);
-      walk.part = P.kv_idx + (size_t)row * P.kv_width;
-    }
-  }
+  const KvWalk walk = make_kv_walk(P, b, h, q0, BN);
   const int n_it = walk.count();
 
   u32x4 kst[GLOADS][4], vst[GLOADS][4];
@@ -477,6 +473,12 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(BwdArgs a) {
         }
       }
   }
+}
+
+template <typename T, int D, int BN, int NW, bool kMods, class Mod = BuiltinMod>
+__global__ __launch_bounds__(NW * 64) void dq_kernel(BwdArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[dq_item_lds<T, D, BN>()];
+  dq_item<T, D, BN, NW, kMods, Mod>(a, lds);
 }
 
 }  // namespace fa

@@ -118,6 +118,19 @@ int bwd_d(const BwdArgs& a, int D, const Tiles& t, int stages, hipStream_t s) {
   }
 }
 
+// compute units of the current device (cached per device)
+int device_cus() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
+
 // Validates the params for the requested backward stages and launches them.
 int bwd_stages(const fa_params* p, BwdArgs& a, int stages, hipStream_t s) {
   if (!p) return FA_ERR_NULL;
@@ -136,6 +149,7 @@ int bwd_stages(const fa_params* p, BwdArgs& a, int stages, hipStream_t s) {
     if ((stages & kStageDq) && !a.p.kv_num && !a.p.full_kv_num) return FA_ERR_TABLES;
     if ((stages & kStageDkdv) && !a.p.q_num && !a.p.full_q_num) return FA_ERR_TABLES;
   }
+  t.ng = fa::f32_groups(p, fa::dq_grid(a.p, t.bm), device_cus());
   const bool m = has_mods(a.p);
   if (p->dtype == FA_DTYPE_BF16)
     return m ? bwd_d<uint16_t, true>(a, p->D, t, stages, s) : bwd_d<uint16_t, false>(a, p->D, t, stages, s);
@@ -168,19 +182,6 @@ int mask_layout(const fa_mask_build* m, MaskLayout* L) {
   L->kdoc_off = L->qdoc_off + up((size_t)m->rows * L->nq * 4);
   L->total = L->kdoc_off + up((size_t)m->rows * L->nk * 4);
   return FA_OK;
-}
-
-// compute units of the current device (cached per device)
-int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 int fwd_launch(const fa_params* p, const fa_kv_cache* kv, const void* q, const void* k, const void* v, void* o,
@@ -224,6 +225,7 @@ int fwd_launch(const fa_params* p, const fa_kv_cache* kv, const void* q, const v
   a.o = o;
   a.lse = lse;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  t.ng = fa::f32_groups(p, fwd_items(a.p, 0, t.bm), device_cus());
   const bool m = has_mods(a.p);
   if (p->dtype == FA_DTYPE_BF16)
     return m ? fwd_d<uint16_t, true>(a, p->D, t, s) : fwd_d<uint16_t, false>(a, p->D, t, s);

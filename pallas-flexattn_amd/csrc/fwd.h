@@ -69,8 +69,39 @@ struct KvTab {
   }
 };
 
-template <typename T, int D, int BN, int NW, bool kMods, class Mod = BuiltinMod>
-__global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
+// The kv walk of the query tile at q0 (tables of (b, h), or every tile).
+__device__ __forceinline__ KvWalk make_kv_walk(const Problem& P, int b, int h, int q0, int bn) {
+  KvWalk walk;
+  walk.bn = bn;
+  walk.mblk = P.mblk_kv;
+  walk.sub = P.mblk_kv / bn;
+  walk.nblk = P.n_kvblk;
+  walk.dense = !P.has_tables;
+  walk.ntiles_dense = (P.Skv + bn - 1) / bn;
+  walk.dense_masked = P.has_mask;
+  walk.full = walk.part = nullptr;
+  walk.nfull = walk.npart = 0;
+  if (P.has_tables) {
+    const int row = tab_row(P, b, h, q0 / P.mblk_q, P.n_qblk);
+    if (P.full_kv_num) {
+      walk.nfull = clamp_count(scalar_load(P.full_kv_num, row), P.kv_width);
+      walk.full = P.full_kv_idx + (size_t)row * P.kv_width;
+    }
+    if (P.kv_num) {
+      walk.npart = clamp_count(scalar_load(P.kv_num, row), P.kv_width);
+      walk.part = P.kv_idx + (size_t)row * P.kv_width;
+    }
+  }
+  return walk;
+}
+
+// One work item of the general forward; `lds`: fwd_item_lds() bytes.
+template <typename T, int D, int BN>
+constexpr int fwd_item_lds() {
+  return 2 * BN * D * (int)sizeof(T);
+}
+template <typename T, int D, int BN, int NW, bool kMods, class Mod>
+__device__ __forceinline__ void fwd_item(const FwdArgs& a, char* lds) {
   using E = Elt<T>;
   using frag = typename E::frag;
   constexpr int BM = 32 * NW;
@@ -88,8 +119,8 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
   using VTile = LdsTile<T, D, BN, 1>;
   static_assert(D % 32 == 0 && BN % 32 == 0, "tile shape");
 
-  __shared__ __attribute__((aligned(16))) char lds_k[KTile::kBytes];
-  __shared__ __attribute__((aligned(16))) char lds_v[VTile::kBytes];
+  char* const lds_k = lds;
+  char* const lds_v = lds + KTile::kBytes;
 
   const Problem& P = a.p;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -114,27 +145,7 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
   const float slope = P.alibi ? P.alibi[h] : 0.f;
   const int qdoc = (P.q_doc && qvalid) ? P.q_doc[(size_t)b * P.Sq + qw] : 0;
 
-  KvWalk walk;
-  walk.bn = BN;
-  walk.mblk = P.mblk_kv;
-  walk.sub = P.mblk_kv / BN;
-  walk.nblk = P.n_kvblk;
-  walk.dense = !P.has_tables;
-  walk.ntiles_dense = (P.Skv + BN - 1) / BN;
-  walk.dense_masked = P.has_mask;
-  walk.full = walk.part = nullptr;
-  walk.nfull = walk.npart = 0;
-  if (P.has_tables) {
-    const int row = tab_row(P, b, h, q0 / P.mblk_q, P.n_qblk);
-    if (P.full_kv_num) {
-      walk.nfull = clamp_count(scalar_load(P.full_kv_num, row), P.kv_width);
-      walk.full = P.full_kv_idx + (size_t)row * P.kv_width;
-    }
-    if (P.kv_num) {
-      walk.npart = clamp_count(scalar_load(P.kv_num, row), P.kv_width);
-      walk.part = P.kv_idx + (size_t)row * P.kv_width;
-    }
-  }
+  const KvWalk walk = make_kv_walk(P, b, h, q0, BN);
   const int n_it = walk.count();
 
   u32x4 kst[KLOADS];
@@ -275,6 +286,12 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
       }
     if (hh == 0) a.lse[(size_t)head * P.Sq + qw] = lt > 0.f ? (m + log2f(lt)) * kLn2 : -INFINITY;
   }
+}
+
+template <typename T, int D, int BN, int NW, bool kMods, class Mod = BuiltinMod>
+__global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[fwd_item_lds<T, D, BN>()];
+  fwd_item<T, D, BN, NW, kMods, Mod>(a, lds);
 }
 
 }  // namespace fa

@@ -2,6 +2,7 @@
 // (FA_KERNELS_D) and one direction (FA_KERNELS_BWD = 0: forward, 1:
 // backward); build.py compiles this file once per pair.
 #include "bwd_bf16.h"
+#include "f32_split.h"
 #include "fwd_bf16.h"
 #include "launch.h"
 
@@ -11,14 +12,23 @@
 
 namespace fa {
 
-// (BN, NW) of the generic kernels: one key tile per dtype, up to 4 waves
-template <typename T, int BN, int NW>
+// (BN, NW) of the generic bf16 kernels (document labels compared per
+// element): one key tile, up to 4 waves.  float32 calls run the split kernels
+// (f32_split.h, 32-key tiles), which fall back to the generic code by
+// themselves.
+template <int BN, int NW>
 constexpr bool generic_tile() {
-  return BN == (sizeof(T) == 2 ? 64 : 32) && NW <= 4;
+  return BN == 64 && NW <= 4;
+}
+
+// float32 forward and dQ launches that two groups of waves can share
+template <int D, int NW>
+constexpr bool f32_grouped() {
+  return D <= 64 && NW == 4;
 }
 
 template <typename T, int D, int BN, int NW, bool M, int NS = 2>
-int run_fwd(const FwdArgs& a, hipStream_t s) {
+int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
   const int grid = fwd_items(a.p, a.pack, 32 * NW);
   if constexpr (sizeof(T) == 2) {
     if (interval_masks(a.p)) {  // bf16: LDS-DMA + transposing-read kernel
@@ -49,10 +59,19 @@ int run_fwd(const FwdArgs& a, hipStream_t s) {
       return launch_status();
     }
   }
-  if constexpr (generic_tile<T, BN, NW>() && NS == 2) {
-    FwdArgs g = a;  // the generic kernel has no split-KV, packed or paged form
-    g.n_splits = 1;
-    g.pack = 0;
+  FwdArgs g = a;  // these have no split-KV, packed or paged form
+  g.n_splits = 1;
+  g.pack = 0;
+  if constexpr (sizeof(T) == 4) {
+    const dim3 items(fwd_items(a.p, 0, 32 * NW));
+    if constexpr (f32_grouped<D, NW>())
+      if (groups == 2) {
+        hipLaunchKernelGGL((fa::fwd_f32_kernel<D, NW, M, fa::BuiltinMod, 2>), items, dim3(2 * NW * 64), 0, s, g);
+        return launch_status();
+      }
+    hipLaunchKernelGGL((fa::fwd_f32_kernel<D, NW, M>), items, dim3(NW * 64), 0, s, g);
+    return launch_status();
+  } else if constexpr (generic_tile<BN, NW>() && NS == 2) {
     hipLaunchKernelGGL((fa::fwd_kernel<T, D, BN, NW, M>), dim3(fwd_items(a.p, 0, 32 * NW)), dim3(NW * 64), 0, s, g);
     return launch_status();
   }
@@ -70,12 +89,12 @@ int launch_fwd(const FwdArgs& a, const Tiles& t, hipStream_t s) {
     }
     return t.bm == 64 ? run_fwd<T, D, 64, 2, M>(a, s) : run_fwd<T, D, 64, 4, M>(a, s);
   } else {
-    return t.bm == 64 ? run_fwd<T, D, 32, 2, M>(a, s) : run_fwd<T, D, 32, 4, M>(a, s);
+    return t.bm == 64 ? run_fwd<T, D, 32, 2, M>(a, s) : run_fwd<T, D, 32, 4, M>(a, s, t.ng);
   }
 }
 
 template <typename T, int D, int BN, int NW, bool M>
-int run_dq(const BwdArgs& a, hipStream_t s) {
+int run_dq(const BwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
   const int grid = dq_grid(a.p, 32 * NW);
   if constexpr (sizeof(T) == 2) {
     if (interval_masks(a.p)) {
@@ -83,7 +102,15 @@ int run_dq(const BwdArgs& a, hipStream_t s) {
       return launch_status();
     }
   }
-  if constexpr (generic_tile<T, BN, NW>()) {
+  if constexpr (sizeof(T) == 4) {
+    if constexpr (f32_grouped<D, NW>())
+      if (groups == 2) {
+        hipLaunchKernelGGL((fa::dq_f32_kernel<D, NW, M, fa::BuiltinMod, 2>), dim3(grid), dim3(2 * NW * 64), 0, s, a);
+        return launch_status();
+      }
+    hipLaunchKernelGGL((fa::dq_f32_kernel<D, NW, M>), dim3(grid), dim3(NW * 64), 0, s, a);
+    return launch_status();
+  } else if constexpr (generic_tile<BN, NW>()) {
     hipLaunchKernelGGL((fa::dq_kernel<T, D, BN, NW, M>), dim3(grid), dim3(NW * 64), 0, s, a);
     return launch_status();
   }
@@ -99,7 +126,13 @@ int run_dkdv(const BwdArgs& a, hipStream_t s) {
       return launch_status();
     }
   }
-  if constexpr (NW == 4 && BQ <= 64) {
+  if constexpr (sizeof(T) == 4) {
+    // at D = 32 two groups fit two waves per SIMD, which one does not reach
+    // (B4 H16 S4096 causal 832 against 1110 us, B4 H8 S1000 58 against 75)
+    constexpr int NG = D == 32 ? 2 : 1;
+    hipLaunchKernelGGL((fa::dkdv_f32_kernel<D, NW, M, fa::BuiltinMod, NG>), dim3(grid), dim3(NG * NW * 64), 0, s, a);
+    return launch_status();
+  } else if constexpr (NW == 4 && BQ <= 64) {
     hipLaunchKernelGGL((fa::dkdv_kernel<T, D, BQ, NW, M>), dim3(grid), dim3(NW * 64), 0, s, a);
     return launch_status();
   }
@@ -116,7 +149,7 @@ int launch_dq(const BwdArgs& a, const Tiles& t, hipStream_t s) {
     }
     return t.bm == 64 ? run_dq<T, D, 64, 2, M>(a, s) : run_dq<T, D, 64, 4, M>(a, s);
   } else {
-    return t.bm == 64 ? run_dq<T, D, 32, 2, M>(a, s) : run_dq<T, D, 32, 4, M>(a, s);
+    return t.bm == 64 ? run_dq<T, D, 32, 2, M>(a, s) : run_dq<T, D, 32, 4, M>(a, s, t.ng);
   }
 }
 

@@ -18,6 +18,7 @@ struct Tiles {
   int bm, bn;    // forward / dQ: query tile, key tile
   int bkv, bq;   // dK/dV: key tile, query tile
   int ns;        // forward: K / V tiles held in LDS (stages)
+  int ng = 1;    // float32 forward / dQ: groups of waves that share a work item (f32_groups)
 };
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -89,6 +90,18 @@ inline int dkdv_query_tile(const fa_params* p, const Problem& pr, Tiles* t) {
   const bool q128 = p->D >= 64 && t->bkv == 128 && interval_masks(pr) && (!pr.has_tables || pr.mblk_q % 128 == 0);
   if (t->bq == 0) t->bq = (q128 && p->D >= 128) ? 128 : 64;
   return (t->bq == 128 && !q128) ? FA_ERR_UNSUPPORTED : FA_OK;
+}
+
+// float32 forward and dQ: a work item's key tiles are shared by two groups of
+// waves where the grid (`items` workgroups) gives a compute unit at most two
+// workgroups, so that the longest walks take half the steps; larger grids fill
+// the SIMDs by themselves and keep the tiles in one group (f32_split.h has no
+// room for two groups at D = 128).  Measured, causal D = 64, one group / two:
+// 256 items (B4 H8 S1000) forward 62 / 47 us, dQ 76 / 61; 512 items 73 / 65
+// and 93 / 86; 1024 items 116 / 127 and 151 / 166; 2048 items (B4 H16 S4096)
+// 732 / 721 and 982 / 1028.
+inline int f32_groups(const fa_params* p, int items, int cus) {
+  return (p->dtype == FA_DTYPE_F32 && p->D <= 64 && items <= 2 * cus) ? 2 : 1;
 }
 
 // Byte budgets of a head group: the L2 of one XCD is 4 MiB; q-tile walks

@@ -41,16 +41,15 @@ struct BlobHeader {
 
 // Kernel instantiations for a policy: the bf16 tile kernels (128-query
 // forward / dQ tiles of 64 keys, 128-key dK/dV tiles of 64 queries) or the
-// generic float32 kernels (32-key tiles).
+// float32 split kernels (32-row tiles).
 std::vector<std::string> mod_kernels(int dtype, int D, bool mods) {
   const std::string d = std::to_string(D), m = mods ? "true" : "false";
   if (dtype == FA_DTYPE_BF16)
     return {"fa::fwd_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>",
             "fa::dq_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>",
             "fa::dkdv_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>"};
-  return {"fa::fwd_kernel<float, " + d + ", 32, 4, " + m + ", UserMod>",
-          "fa::dq_kernel<float, " + d + ", 32, 4, " + m + ", UserMod>",
-          "fa::dkdv_kernel<float, " + d + ", 32, 4, " + m + ", UserMod>"};
+  return {"fa::fwd_f32_kernel<" + d + ", 4, " + m + ", UserMod>", "fa::dq_f32_kernel<" + d + ", 4, " + m + ", UserMod>",
+          "fa::dkdv_f32_kernel<" + d + ", 4, " + m + ", UserMod>"};
 }
 
 void copy_log(const std::string& text, char* log, size_t log_bytes) {
@@ -73,7 +72,7 @@ int compile_mods(const char* policy, int dtype, int D, int flags, std::vector<ch
   const bool mods = (flags & (FA_MODS_SCORE | FA_MODS_BUILTIN_SCORE)) != 0;
   const std::vector<std::string> kernels = mod_kernels(dtype, D, mods);
   std::string src = dtype == FA_DTYPE_BF16 ? "#include \"fwd_bf16.h\"\n#include \"bwd_bf16.h\"\n"
-                                           : "#include \"fwd.h\"\n#include \"bwd.h\"\n";
+                                           : "#include \"f32_split.h\"\n";
   src += "\n";
   src += policy;
   src += "\n";

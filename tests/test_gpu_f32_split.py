@@ -1,0 +1,64 @@
+"""The float32 kernels' split products (three bf16 pieces per operand) at the edges of their tiles, with
+one and two groups of waves per work item, and on inputs that take the float32 matrix instructions
+instead (magnitudes from 2^30, infinities)."""
+import numpy as np
+import pytest
+
+from _cases import FP32_TOL, assert_close, inputs, oracle_fwd_bwd, to_np, to_torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(pf, q, k, v, do, mask, tiles=None):
+    import torch
+    q, k, v, do = (to_torch(x, "fp32") for x in (q, k, v, do))
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    bm = None if mask is None else pf.create_block_mask(mask, q.shape[0], q.shape[1], q.shape[2], k.shape[2], 128)
+    opts = None if tiles is None else {"BLOCK_M": tiles}
+    o = pf.flex_attention(q, k, v, block_mask=bm, enable_gqa=q.shape[1] != k.shape[1], kernel_options=opts)
+    return [to_np(x) for x in (o.detach(),) + torch.autograd.grad(o, (q, k, v), do)]
+
+
+# one and two groups: at most 512 work items share theirs between two (256 CUs), B 9 H 64 has 576 and more
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,tiles", [
+    (1, 2, 2, 1, 1, 64, False, None), (1, 2, 1, 33, 31, 32, False, None), (1, 2, 2, 127, 127, 64, True, None),
+    (1, 2, 2, 129, 129, 128, True, None), (2, 2, 1, 257, 257, 64, True, None), (1, 2, 2, 95, 289, 64, False, None),
+    (1, 2, 2, 200, 200, 128, True, 64), (1, 2, 2, 160, 160, 32, True, 64), (9, 64, 64, 40, 40, 32, True, None),
+    (9, 64, 32, 33, 65, 64, False, None)])
+def test_tile_edges(B, Hq, Hkv, Sq, Skv, D, causal, tiles):
+    import pallas_flexattn as pf
+    q, k, v, do = inputs(31 + Sq, B, Hq, Hkv, Sq, Skv, D, "fp32")
+    got = _run(pf, q, k, v, do, pf.causal_mask if causal else None, tiles)
+    dense = np.broadcast_to(np.tril(np.ones((Sq, Skv), bool)) if causal else np.ones((Sq, Skv), bool),
+                            (B, Hq, Sq, Skv))
+    o, _, grads = oracle_fwd_bwd(q, k, v, do, dense)
+    for name, a, b in zip("o dq dk dv".split(), got, (o,) + tuple(grads)):
+        assert_close(name, a, b, FP32_TOL)
+
+
+@pytest.mark.parametrize("S,D", [(70, 64), (300, 64), (130, 128)])
+def test_large_and_infinite_inputs_take_the_float32_instructions(S, D):
+    import pallas_flexattn as pf
+    rng = np.random.default_rng(5)
+    q, k, v, do = (rng.standard_normal((1, 2, S, D)).astype(np.float32) for _ in range(4))
+    v[0, 0, 3, 7] = np.inf   # every row sees key 3: column 7 of head 0 is inf, the rest as without it
+    v[0, 1, 5, 2] = 3.0e38   # no bf16 piece holds it
+    k[0, 1, 9] = 0.0
+    q[0, 1, 4] *= 2.0 ** 31  # a one-hot row in the limit; its scores are far apart
+    o = _run_fwd(pf, q, k, v)
+    s = q.astype(np.float64) @ k.astype(np.float64).transpose(0, 1, 3, 2) / np.sqrt(D)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    vf = np.where(np.isinf(v), 0.0, v).astype(np.float64)
+    want = p @ vf
+    assert np.all(np.isposinf(o[0, 0, :, 7]))
+    got = o.astype(np.float64)
+    got[0, 0, :, 7] = want[0, 0, :, 7]
+    # per element, relative to the magnitudes summed (3e38 in one column)
+    scale = p @ np.abs(vf)
+    assert np.max(np.abs(got - want) / scale) < 1e-5
+
+
+def _run_fwd(pf, q, k, v):
+    return to_np(pf.flex_attention(*(to_torch(x, "fp32") for x in (q, k, v))))
