@@ -213,7 +213,12 @@ int fwd_launch(const fa_params* p, const fa_kv_cache* kv, const void* q, const v
     a.kv_lens = kv->kv_lens;
   }
   a.pack = choose_pack(p, t, a.p);
-  a.n_splits = split ? choose_splits(p, t, a.p, n_splits, device_cus()) : 1;
+  const bool lens = kv && kv->kv_lens;
+  a.n_splits = split ? choose_splits(p, t, a.p, n_splits, device_cus(), lens) : 1;
+  a.split_keys = fa::choose_split_keys(p, a.p, a.n_splits, lens);
+  // rows of different lengths: an XCD that took whole batch rows (the L2 order)
+  // would get more or less work than the others, so the heads go round the XCDs
+  if (lens && fa::one_wave_fwd(a.p, a.pack, p->D)) a.p.xcd_remap = 0;
   if (a.n_splits > 1) {
     if (!workspace || workspace_bytes < split_bytes(p, a.n_splits) || !aligned16({workspace}))
       return FA_ERR_WORKSPACE;
@@ -265,7 +270,10 @@ size_t fa_fwd_splitkv_workspace_bytes(const fa_params* p, int n_splits) {
   Problem pr;
   if (!p || default_tiles(p, &t) || build_problem(p, t, &pr)) return 0;
   if (n_splits > 64) return 0;
-  return split_bytes(p, choose_splits(p, t, pr, n_splits, device_cus()));
+  // (enough for a call with or without per-row lengths)
+  const int cus = device_cus();
+  return split_bytes(p, fa::imax(choose_splits(p, t, pr, n_splits, cus, false),
+                                 choose_splits(p, t, pr, n_splits, cus, true)));
 }
 
 int fa_fwd_splitkv(const fa_params* p, const void* q, const void* k, const void* v, void* o, float* lse,

@@ -29,7 +29,10 @@ struct FwdArgs {
   // split blockIdx.x / items of its item's walk and writes, instead of o and
   // lse, its unnormalised partial O (relative to 2^m) and (m, l) to `part`:
   // (n_splits, B*Hq*Sq, D) floats, then (n_splits, B*Hq*Sq, 2).
+  // A split takes an equal share of the walk, or with split_keys > 0 (a
+  // multiple of 64) the tiles of its split_keys keys, none past a row's length.
   int n_splits = 1;
+  int split_keys = 0;
   float* part = nullptr;
   // bf16 DMA kernel only:
   // GQA row packing (pack > 1): a work item is (batch, kv head, BM rows) of

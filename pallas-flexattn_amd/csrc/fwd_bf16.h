@@ -158,6 +158,20 @@ void fwd_bf16_kernel(FwdArgs a) {
     }
   }
   const int n_it = walk.count();
+  [[maybe_unused]] const int chunk = a.split_keys / BN;
+  // a split past a short row's keys has nothing to read: (m, l) = (-inf, 0),
+  // its partial O is never looked at
+  if constexpr (kCache) {
+    const SplitRange sr = split_range(n_it, split, a.n_splits, chunk);
+    if (a.n_splits > 1 && sr.it0 >= sr.it1) {
+      if (qvalid && hh == 0) {
+        const size_t all_rows = (size_t)P.B * P.Hq * P.Sq;
+        float* pml = a.part + (size_t)a.n_splits * all_rows * D + ((size_t)split * all_rows + row0 + rw) * 2;
+        *reinterpret_cast<float2*>(pml) = make_float2(-INFINITY, 0.f);
+      }
+      return;
+    }
+  }
 
   // HBM -> LDS copies of the tile starting at key kb into buffer `buf`: the
   // resources (issue_plan), then the 2 * IPW copy instructions one at a time
@@ -285,8 +299,15 @@ void fwd_bf16_kernel(FwdArgs a) {
   // measured against a table load per tile).
   // With split-KV this workgroup takes tiles [it0, it1) of the walk.
   const int n_full = walk.count_full();
-  const int it0 = a.n_splits > 1 ? (int)((long long)n_it * split / a.n_splits) : 0;
-  const int it1 = a.n_splits > 1 ? (int)((long long)n_it * (split + 1) / a.n_splits) : n_it;
+  int it0, it1;
+  if constexpr (kCache) {
+    const SplitRange sr = split_range(n_it, split, a.n_splits, chunk);
+    it0 = sr.it0;
+    it1 = sr.it1;
+  } else {  // equal shares, written out: the shared form costs the unsplit forward 0.7 % (SGPR layout)
+    it0 = a.n_splits > 1 ? (int)((long long)n_it * split / a.n_splits) : 0;
+    it1 = a.n_splits > 1 ? (int)((long long)n_it * (split + 1) / a.n_splits) : n_it;
+  }
   const int sub_log2 = log2_if_pow2(walk.sub);
   KvTab tab;
   auto kbase_of = [&](int it) { return tab.kbase(walk, it, sub_log2, lane); };
@@ -511,33 +532,80 @@ void fwd_bf16_kernel(FwdArgs a) {
   if (qvalid && hh == 0) a.lse[row0 + rw] = lt > 0.f ? (m + log2f(lt)) * kLn2 : -INFINITY;
 }
 
-// Split-KV merge: one thread per (row, column) of O.  With the splits'
-// partials O_s (relative to 2^m_s) and sums l_s: M = max m_s, L = sum l_s
-// 2^(m_s - M), O = sum O_s 2^(m_s - M) / L, LSE = (M + log2 L) ln 2.
-template <int D>
+// Split-KV merge.  With the splits' partials O_s (relative to 2^m_s) and sums
+// l_s: M = max m_s, L = sum l_s 2^(m_s - M), O = sum O_s 2^(m_s - M) / L,
+// LSE = (M + log2 L) ln 2.  One wave per row takes up to 16 splits (lane s
+// holds split s's factor, the columns go over the lanes, loads eight splits
+// deep); with more, the four waves of a workgroup share one row's splits and
+// add up through LDS.  Bound by latency: a thread per element that walked the
+// splits one load at a time took 6.8 us for 256 rows of 8 splits and 20 us for
+// 32 rows of 64, this 3.1 and 4.5.
+template <int D, bool kShared>
 __global__ __launch_bounds__(256) void fwd_split_merge(FwdArgs a) {
+  constexpr int CPL = D >= 64 ? D / 64 : 1;  // columns per lane
+  __shared__ float sums[kShared ? 4 * D : 1];
   const Problem& P = a.p;
   const size_t rows = (size_t)P.B * P.Hq * P.Sq;
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const size_t row = idx / D;
-  const int d = (int)(idx - row * D);
-  if (row >= rows) return;
-  const float* pml = a.part + (size_t)a.n_splits * rows * D;
-  float mm = -INFINITY;
-  for (int s = 0; s < a.n_splits; ++s) mm = fmaxf(mm, pml[((size_t)s * rows + row) * 2]);
-  float L = 0.f, O = 0.f;
-  if (mm != -INFINITY) {
-    for (int s = 0; s < a.n_splits; ++s) {
-      const float ms = pml[((size_t)s * rows + row) * 2];
-      const float c = ms == -INFINITY ? 0.f : fast_exp2(ms - mm);
-      L += pml[((size_t)s * rows + row) * 2 + 1] * c;
-      O += a.part[((size_t)s * rows + row) * D + d] * c;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const size_t row = kShared ? (size_t)blockIdx.x : (size_t)blockIdx.x * 4 + w;
+  if (row >= rows) return;  // (wave-uniform; with kShared the grid has one workgroup per row)
+  const int n = a.n_splits;
+  const float* pml = a.part + (size_t)n * rows * D;
+  float2 ml = make_float2(-INFINITY, 0.f);
+  if (lane < n) ml = *reinterpret_cast<const float2*>(pml + ((size_t)lane * rows + row) * 2);
+  float mm = ml.x;
+#pragma unroll
+  for (int x = 32; x >= 1; x >>= 1) mm = fmaxf(mm, __shfl_xor(mm, x, 64));
+  const float c = ml.x == -INFINITY ? 0.f : fast_exp2(ml.x - mm);
+  float L = ml.y * c;
+#pragma unroll
+  for (int x = 32; x >= 1; x >>= 1) L += __shfl_xor(L, x, 64);
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  const int col = lane * CPL < D ? lane * CPL : 0;  // (D = 32: lanes 32 .. 63 repeat column 0)
+  float acc[CPL];
+#pragma unroll
+  for (int k = 0; k < CPL; ++k) acc[k] = 0.f;
+  const float* po = a.part + row * D + col;
+  constexpr int STEP = kShared ? 4 : 1, DEEP = 8;
+  for (int s0 = kShared ? w : 0; s0 < n; s0 += STEP * DEEP) {
+    float x[DEEP][CPL];
+#pragma unroll
+    for (int u = 0; u < DEEP; ++u) {
+      const int s = imin(s0 + u * STEP, n - 1);
+      const float* p = po + (size_t)s * rows * D;
+      if constexpr (CPL == 2) {
+        const float2 v = *reinterpret_cast<const float2*>(p);
+        x[u][0] = v.x;
+        x[u][1] = v.y;
+      } else {
+        x[u][0] = p[0];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < DEEP; ++u) {
+      const int s = s0 + u * STEP;
+      // a split without a live key left its partial O unwritten
+      const float cs = __shfl(c, s & 63, 64);
+      const bool live = s < n && !(cs == 0.f);  // (NaN is passed on)
+#pragma unroll
+      for (int k = 0; k < CPL; ++k) acc[k] = live ? fmaf(x[u][k], cs, acc[k]) : acc[k];
     }
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
-  const uint32_t ob = pack_bf16x2(O * inv, 0.f);
-  static_cast<uint16_t*>(a.o)[row * D + d] = (uint16_t)(ob & 0xffffu);
-  if (d == 0) a.lse[row] = L > 0.f ? (mm + log2f(L)) * kLn2 : -INFINITY;
+  if constexpr (kShared) {
+#pragma unroll
+    for (int k = 0; k < CPL; ++k)
+      if (lane * CPL < D) sums[w * D + col + k] = acc[k];
+    __syncthreads();
+    if (w) return;
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) acc[k] = (sums[col + k] + sums[D + col + k]) + (sums[2 * D + col + k] + sums[3 * D + col + k]);
+  }
+  if (lane * CPL < D) {
+    uint16_t* o = static_cast<uint16_t*>(a.o) + row * D + col;
+    if constexpr (CPL == 2) *reinterpret_cast<uint32_t*>(o) = pack_bf16x2(acc[0] * inv, acc[1] * inv);
+    else *o = (uint16_t)(pack_bf16x2(acc[0] * inv, 0.f) & 0xffffu);
+  }
+  if (lane == 0) a.lse[row] = L > 0.f ? (mm + log2f(L)) * kLn2 : -INFINITY;
 }
 
 }  // namespace fa

@@ -241,6 +241,20 @@ FA_HD PageSpan page_span(int kb, int pg, int skv, int page_size, int phys, int n
   return PageSpan{row, ok ? imin(page_size - off, skv - kb) : 0};
 }
 
+// Tiles [it0, it1) of an n_it-tile walk that split `split` of n_splits takes:
+// runs of `chunk` tiles, or with chunk = 0 equal shares of the walk.
+struct SplitRange {
+  int it0, it1;
+};
+FA_HD SplitRange split_range(int n_it, int split, int n_splits, int chunk) {
+  if (n_splits <= 1) return SplitRange{0, n_it};
+  if (chunk > 0) {
+    const int it0 = imin(split * chunk, n_it);
+    return SplitRange{it0, imin(it0 + chunk, n_it)};
+  }
+  return SplitRange{(int)((long long)n_it * split / n_splits), (int)((long long)n_it * (split + 1) / n_splits)};
+}
+
 // A tile of a walk whose table entry may still be in flight: fetch() issues
 // the load, the walk's resolve step turns the entry into a tile start (an
 // iteration or two later, so the load latency is hidden).

@@ -34,14 +34,14 @@ int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
     if (interval_masks(a.p)) {  // bf16: LDS-DMA + transposing-read kernel
       const bool cache = a.pack > 1 || a.page_table || a.kv_lens;
       if constexpr (NW == 4 && BN == 64) {
-        // split-KV decode (every packed row in one 32-row block): one wave
+        // split-KV decode (every row of an item in one 32-row block): one wave
         // per workgroup and 32-key tiles, 4x less MFMA work on dead rows and
         // half the LDS per workgroup; measured 5.72 against 5.40 TB/s of KV
         // reads at B8 Hq32 Hkv8 Skv32768 (a plain streaming read reaches
         // ~5.8).  Unsplit, its grid of one-wave workgroups is too small.
-        if (cache && a.pack > 1 && a.pack * a.p.Sq <= 32 && a.n_splits > 1 && D >= 64)
-          hipLaunchKernelGGL((fa::fwd_bf16_kernel<D, 32, 1, M, fa::BuiltinMod, true>), dim3(grid * a.n_splits),
-                             dim3(64), 0, s, a);
+        if (one_wave_fwd(a.p, a.pack, D) && a.n_splits > 1)
+          hipLaunchKernelGGL((fa::fwd_bf16_kernel<D, 32, 1, M, fa::BuiltinMod, true>),
+                             dim3(fwd_items(a.p, a.pack, 32) * a.n_splits), dim3(64), 0, s, a);
         else if (cache)
           hipLaunchKernelGGL((fa::fwd_bf16_kernel<D, BN, NW, M, fa::BuiltinMod, true>), dim3(grid * a.n_splits),
                              dim3(NW * 64), 0, s, a);
@@ -53,8 +53,11 @@ int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
                            dim3(NW * 64), 0, s, a);
       }
       if (a.n_splits > 1) {
-        const size_t n = (size_t)a.p.B * a.p.Hq * a.p.Sq * D;
-        hipLaunchKernelGGL((fa::fwd_split_merge<D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
+        const unsigned rows = (unsigned)a.p.B * a.p.Hq * a.p.Sq;
+        if (a.n_splits > 16)
+          hipLaunchKernelGGL((fa::fwd_split_merge<D, true>), dim3(rows), dim3(256), 0, s, a);
+        else
+          hipLaunchKernelGGL((fa::fwd_split_merge<D, false>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
       }
       return launch_status();
     }

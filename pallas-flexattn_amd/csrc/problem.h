@@ -202,18 +202,42 @@ inline int choose_pack(const fa_params* p, const Tiles& t, const Problem& pr) {
   return g;
 }
 
-// Split-KV: the requested count (<= 0: about two workgroups per CU of the
-// cus compute units, at least four key tiles per split), or 1 where the
-// generic kernel runs.
-inline int choose_splits(const fa_params* p, const Tiles& t, const Problem& pr, int requested, int cus) {
+// Decode shapes: every row of a work item in one 32-row block (g * Sq packed
+// rows, or Sq), which the split forward runs as one wave per workgroup.
+inline bool one_wave_fwd(const Problem& pr, int pack, int D) {
+  return D >= 64 && (pack > 1 ? pack : 1) * pr.Sq <= 32;
+}
+
+// Split-KV: the requested count, or 1 where the generic kernel runs.  <= 0:
+// as many as give a CU (of cus) two workgroups, at least four key tiles per
+// split.  The one-wave workgroups of decode shapes take more: a tile in flight
+// is half as many bytes at D = 64 (four: B16 Hq32 Hkv4 Skv8192 27 us against
+// 40 with one, 27 with two to eight; B6 H4 Skv16640 21 against 25 with two),
+// and rows of different lengths (`lens`) balance over five (B32 Hq32 Hkv8
+// Skv8192 D128, lengths of a tenth and more: 144 / 115 / 104 / 122 us with 2 /
+// 3 / 5 / 8; B18 Hq128 Hkv16 Skv10368 D64 160 / 118 / 91 / 100).  With equal
+// lengths at D = 128 more than two only cost merging (B8 Hq32 Hkv8 Skv32768:
+// 184 / 191 / 205 us with 2 / 3 / 6).
+inline int choose_splits(const fa_params* p, const Tiles& t, const Problem& pr, int requested, int cus, bool lens) {
   if (p->dtype != FA_DTYPE_BF16 || !interval_masks(pr)) return 1;
-  const int items = fwd_items(pr, choose_pack(p, t, pr), t.bm);
+  const int pack = choose_pack(p, t, pr);
+  const int items = fwd_items(pr, pack, t.bm);
   const int max_by_keys = cdiv(p->Skv, 4 * t.bn);
+  const int per_cu = !one_wave_fwd(pr, pack, p->D) ? 2 : lens ? 5 : p->D < 128 ? 4 : 2;
   int n = requested;
-  if (n <= 0) n = cdiv(2 * cus, items);
+  if (n <= 0) n = cdiv(per_cu * cus, items);
   if (n > max_by_keys) n = max_by_keys;
   if (n > 64) n = 64;
   return n < 1 ? 1 : n;
+}
+
+// Keys per split where the rows of a batch have lengths of their own and the
+// walk is dense: equal runs of keys, so that a long row is cut into as many
+// pieces as it needs and no workgroup gets more than the others (104 against
+// 116 us at the first shape above); 0: equal shares of each row's walk.
+inline int choose_split_keys(const fa_params* p, const Problem& pr, int n_splits, bool lens) {
+  if (n_splits <= 1 || !lens || pr.has_tables) return 0;
+  return cdiv(cdiv(p->Skv, n_splits), 64) * 64;
 }
 
 inline size_t split_bytes(const fa_params* p, int n) {

@@ -146,7 +146,7 @@ static bool read_case(FILE* f, Case& c) {
 
 // ---- forward (fwd_bf16_kernel) -------------------------------------------
 struct FwdOpts {
-  int pack = 0, n_splits = 1;
+  int pack = 0, n_splits = 1, split_keys = 0;
   const int* page_table = nullptr;
   int page_size = 0, max_pages = 0, num_pages = 0;
   const int* kv_lens = nullptr;
@@ -254,8 +254,12 @@ static void model_fwd(const Problem& P, const FwdOpts& o) {
       }
     }
     const int n_it = walk.count();
-    const int it0 = o.n_splits > 1 ? (int)((long long)n_it * split / o.n_splits) : 0;
-    const int it1 = o.n_splits > 1 ? (int)((long long)n_it * (split + 1) / o.n_splits) : n_it;
+    const SplitRange sr = split_range(n_it, split, o.n_splits, o.split_keys / BN);
+    const int it0 = sr.it0, it1 = sr.it1;
+    // the splits of an item cover its walk, in order, without overlap
+    if (split == 0 && it0 != 0) fail("first split does not start the walk");
+    if (split == o.n_splits - 1 && it1 != n_it) fail("last split does not end the walk");
+    if (split > 0 && split_range(n_it, split - 1, o.n_splits, o.split_keys / BN).it1 != it0) fail("splits leave a gap");
     const long long head_kv = (long long)(b * P.Hkv + hk) * P.Skv;
     for (int it = it0; it < it1; ++it) {
       const int kb = walk.kbase(walk.fetch(it));
@@ -434,6 +438,7 @@ static void model_dkdv(const Problem& P) {
 template <int D>
 static void run_fwd(const Problem& P, const Tiles& t, const FwdOpts& o) {
   if constexpr (D >= 64) {
+    if (o.n_splits > 1 && one_wave_fwd(P, o.pack, D) && t.bn == 64 && t.bm == 128) return model_fwd<D, 32, 1, 2>(P, o);
     if (t.bn == 32) return t.ns == 3 ? model_fwd<D, 32, 4, 3>(P, o) : model_fwd<D, 32, 4, 2>(P, o);
     if (t.bn == 128) return t.ns == 1 ? model_fwd<D, 128, 4, 1>(P, o) : model_fwd<D, 128, 4, 2>(P, o);
     if (t.bm == 256) return model_fwd<D, 64, 8, 2>(P, o);
@@ -492,7 +497,7 @@ static int check_case(Case& c) {
     // split-KV and GQA packing as the C ABI would choose them (a 256-CU device)
     if (t.bm == 128 && t.bn == 64 && t.ns == 2) {
       o.pack = choose_pack(&p, t, P);
-      o.n_splits = choose_splits(&p, t, P, 0, 256);
+      o.n_splits = choose_splits(&p, t, P, 0, 256, false);
       g_where = "split-KV forward";
       if (c.D == 32) run_fwd<32>(P, t, o); else if (c.D == 64) run_fwd<64>(P, t, o); else run_fwd<128>(P, t, o);
       ++launches;
@@ -537,7 +542,8 @@ static int check_paged(const Case& c) {
   if (build_problem(&p, t, &P) != FA_OK) return 0;
   FwdOpts o;
   o.pack = choose_pack(&p, t, P);
-  o.n_splits = choose_splits(&p, t, P, 0, 256);
+  o.n_splits = choose_splits(&p, t, P, 0, 256, true);
+  o.split_keys = choose_split_keys(&p, P, o.n_splits, true);
   o.page_table = pt;
   o.page_size = ps;
   o.max_pages = maxp;

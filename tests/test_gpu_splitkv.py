@@ -206,3 +206,29 @@ def test_kv_cache_lengths_and_pages(paged):
         o_r, lse_r = pf.flex_decode(q, k, v, enable_gqa=True, kv_lens=kv_lens, num_splits=splits, return_lse=True)
         torch.cuda.synchronize()
         assert torch.equal(o_p, o_r) and torch.equal(lse_p, lse_r), f"paged != contiguous (splits={splits})"
+
+
+@pytest.mark.parametrize("Hq,Hkv,Sq,D,lens,splits", [
+    (8, 2, 1, 128, [0, 1, 63, 64, 65, 2048], None),    # packed rows, one wave per workgroup, 5 workgroups per CU
+    (4, 4, 1, 64, [1, 255, 256, 257, 2047, 2048], None),  # one query row per workgroup
+    (4, 4, 4, 128, [300, 2048, 1, 0, 2000, 129], 64),  # splits past a row's keys; more than 16 to merge
+    (8, 2, 1, 64, [2048, 5, 700, 64, 1024, 1025], 17), (8, 2, 1, 128, [2048, 5, 700, 64, 1024, 1025], 16),
+    (8, 2, 16, 128, [2048, 33, 700, 64, 1024, 1025], None),  # 64 packed rows: the four-wave kernel
+    (4, 2, 1, 32, [2048, 33, 700, 64, 0, 1025], 20)])
+def test_rows_of_different_lengths(Hq, Hkv, Sq, D, lens, splits):
+    """Splits of equal key runs (kv_lens): rows that end inside, at and before a run, empty rows, and
+    both merge forms, against the oracle; a row without keys gives O = 0, LSE = -inf."""
+    import torch
+    import pallas_flexattn as pf
+    B, Skv = len(lens), 2048
+    q, k, v = _case(B, Hq, Hkv, Sq, Skv, D, 11)
+    o, lse = pf.flex_decode(q, k, v, enable_gqa=Hq != Hkv, kv_lens=torch.tensor(lens, dtype=torch.int32),
+                            num_splits=splits, return_lse=True)
+    o, lse = o.float().cpu().numpy(), lse.cpu().numpy()
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert not np.any(o[b]) and np.all(np.isneginf(lse[b]))
+            continue
+        wo, wl = _oracle(q[b:b + 1], k[b:b + 1, :, :n], v[b:b + 1, :, :n])
+        np.testing.assert_allclose(o[b:b + 1], wo, atol=2e-2, rtol=2e-2)
+        np.testing.assert_allclose(lse[b:b + 1], wl, atol=1e-3, rtol=1e-3)
