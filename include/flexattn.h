@@ -180,6 +180,9 @@ typedef struct fa_fp8_inputs {
   const float *q_scale, *k_scale, *v_scale;
 } fa_fp8_inputs;
 int fa_fwd_fp8(const fa_params *p, const fa_fp8_inputs *in, void *o, float *lse, void *stream);
+/* The same with in->q in bf16 (q_scale unused): the forward quantises its Q
+ * rows itself, to the codes and scales fa_quantize_fp8 gives. */
+int fa_fwd_fp8_q16(const fa_params *p, const fa_fp8_inputs *in, void *o, float *lse, void *stream);
 
 /* bf16 rows -> e4m3 with one power-of-two scale per 128-row block:
  * x (heads, S, D) bf16; scale (heads, ceil(S / 128)) = 2^e with e the
@@ -190,6 +193,10 @@ int fa_fwd_fp8(const fa_params *p, const fa_fp8_inputs *in, void *o, float *lse,
  * zero.  D = 32, 64 or 128.  No reference counterpart. */
 int fa_quantize_fp8(const void *x, int32_t heads, int32_t S, int32_t D, int32_t transpose, void *out, float *scale,
                     void *stream);
+/* K and V (heads, S, D) in one launch: k row-major, v transposed, as two calls
+ * of fa_quantize_fp8. */
+int fa_quantize_fp8_kv(const void *k, const void *v, int32_t heads, int32_t S, int32_t D, void *k_out, float *k_scale,
+                       void *vt_out, float *v_scale, void *stream);
 
 /* Host twins of fa_fwd, fa_bwd_preprocess, fa_bwd_dkdv, fa_bwd_dq and fa_bwd:
  * the same params and results on HOST memory, computed by C++ threads (all

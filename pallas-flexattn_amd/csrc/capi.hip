@@ -237,6 +237,38 @@ int fwd_launch(const fa_params* p, const fa_kv_cache* kv, const void* q, const v
   return m ? fwd_d<float, true>(a, p->D, t, s) : fwd_d<float, false>(a, p->D, t, s);
 }
 
+int fwd_fp8_launch(const fa_params* p, const fa_fp8_inputs* in, bool q16, void* o, float* lse, void* stream) {
+  if (!p || !in) return FA_ERR_NULL;
+  (void)device_scratch();
+  if (p->dtype != FA_DTYPE_FP8_E4M3) return FA_ERR_DTYPE;
+  Tiles t;
+  int rc = default_tiles(p, &t);
+  if (rc) return rc;
+  fa::Fp8FwdArgs a;
+  rc = build_problem(p, t, &a.p);
+  if (rc) return rc;
+  if (p->D != 64 && p->D != 128) return FA_ERR_UNSUPPORTED;
+  if (!interval_masks(a.p)) return FA_ERR_UNSUPPORTED;  // document labels: contiguous runs only
+  if (!in->q || !in->k || !in->vt || (!in->q_scale && !q16) || !in->k_scale || !in->v_scale || !o || !lse) return FA_ERR_NULL;
+  if (!aligned16({in->q, in->k, in->vt, o})) return FA_ERR_SHAPE;
+  if (in->v_ld < p->Skv || in->v_ld % 128) return FA_ERR_SHAPE;
+  if ((long long)p->D * in->v_ld > 0xffffffffll || (long long)p->Skv * p->D > 0xffffffffll ||
+      (long long)p->Sq * p->D * (q16 ? 2 : 1) > 0xffffffffll)
+    return FA_ERR_SHAPE;  // one head's rows within a 32-bit buffer range
+  if (a.p.has_tables && (a.p.mblk_q % t.bm || a.p.mblk_kv % t.bn)) return FA_ERR_TABLES;
+  if (a.p.has_tables && !a.p.kv_num && !a.p.full_kv_num) return FA_ERR_TABLES;
+  a.q = static_cast<const uint8_t*>(in->q);
+  a.k = static_cast<const uint8_t*>(in->k);
+  a.vt = static_cast<const uint8_t*>(in->vt);
+  a.ldv = in->v_ld;
+  a.q_scale = in->q_scale;
+  a.k_scale = in->k_scale;
+  a.v_scale = in->v_scale;
+  a.o = o;
+  a.lse = lse;
+  return fa::launch_fwd_fp8(a, p->D, has_mods(a.p), q16, static_cast<hipStream_t>(stream));
+}
+
 #include "user_mods.h"
 
 }  // namespace
@@ -287,35 +319,11 @@ int fa_fwd(const fa_params* p, const void* q, const void* k, const void* v, void
 }
 
 int fa_fwd_fp8(const fa_params* p, const fa_fp8_inputs* in, void* o, float* lse, void* stream) {
-  if (!p || !in) return FA_ERR_NULL;
-  (void)device_scratch();
-  if (p->dtype != FA_DTYPE_FP8_E4M3) return FA_ERR_DTYPE;
-  Tiles t;
-  int rc = default_tiles(p, &t);
-  if (rc) return rc;
-  fa::Fp8FwdArgs a;
-  rc = build_problem(p, t, &a.p);
-  if (rc) return rc;
-  if (p->D != 64 && p->D != 128) return FA_ERR_UNSUPPORTED;
-  if (!interval_masks(a.p)) return FA_ERR_UNSUPPORTED;  // document labels: contiguous runs only
-  if (!in->q || !in->k || !in->vt || !in->q_scale || !in->k_scale || !in->v_scale || !o || !lse) return FA_ERR_NULL;
-  if (!aligned16({in->q, in->k, in->vt, o})) return FA_ERR_SHAPE;
-  if (in->v_ld < p->Skv || in->v_ld % 128) return FA_ERR_SHAPE;
-  if ((long long)p->D * in->v_ld > 0xffffffffll || (long long)p->Skv * p->D > 0xffffffffll ||
-      (long long)p->Sq * p->D > 0xffffffffll)
-    return FA_ERR_SHAPE;  // one head's rows within a 32-bit buffer range
-  if (a.p.has_tables && (a.p.mblk_q % t.bm || a.p.mblk_kv % t.bn)) return FA_ERR_TABLES;
-  if (a.p.has_tables && !a.p.kv_num && !a.p.full_kv_num) return FA_ERR_TABLES;
-  a.q = static_cast<const uint8_t*>(in->q);
-  a.k = static_cast<const uint8_t*>(in->k);
-  a.vt = static_cast<const uint8_t*>(in->vt);
-  a.ldv = in->v_ld;
-  a.q_scale = in->q_scale;
-  a.k_scale = in->k_scale;
-  a.v_scale = in->v_scale;
-  a.o = o;
-  a.lse = lse;
-  return fa::launch_fwd_fp8(a, p->D, has_mods(a.p), static_cast<hipStream_t>(stream));
+  return fwd_fp8_launch(p, in, false, o, lse, stream);
+}
+
+int fa_fwd_fp8_q16(const fa_params* p, const fa_fp8_inputs* in, void* o, float* lse, void* stream) {
+  return fwd_fp8_launch(p, in, true, o, lse, stream);
 }
 
 int fa_quantize_fp8(const void* x, int32_t heads, int32_t S, int32_t D, int32_t transpose, void* out, float* scale,
@@ -325,15 +333,31 @@ int fa_quantize_fp8(const void* x, int32_t heads, int32_t S, int32_t D, int32_t 
   if (D != 32 && D != 64 && D != 128) return FA_ERR_UNSUPPORTED;
   if (!aligned16({x, out})) return FA_ERR_SHAPE;
   if ((long long)heads * cdiv(S, fa::kFp8ScaleRows) > 0x7fffffffll) return FA_ERR_SHAPE;
-  fa::QuantArgs a;
-  a.x = static_cast<const uint16_t*>(x);
-  a.out = static_cast<uint8_t*>(out);
-  a.scale = scale;
+  fa::QuantArgs a{};
+  a.t[0] = {static_cast<const uint16_t*>(x), static_cast<uint8_t*>(out), scale, transpose};
+  a.count = 1;
   a.heads = heads;
   a.S = S;
   a.D = D;
   a.ld = cdiv(S, fa::kFp8ScaleRows) * fa::kFp8ScaleRows;
-  a.transpose = transpose;
+  return fa::launch_quant_fp8(a, static_cast<hipStream_t>(stream));
+}
+
+int fa_quantize_fp8_kv(const void* k, const void* v, int32_t heads, int32_t S, int32_t D, void* k_out, float* k_scale,
+                       void* vt_out, float* v_scale, void* stream) {
+  if (!k || !v || !k_out || !k_scale || !vt_out || !v_scale) return FA_ERR_NULL;
+  if (heads < 1 || S < 1) return FA_ERR_SHAPE;
+  if (D != 32 && D != 64 && D != 128) return FA_ERR_UNSUPPORTED;
+  if (!aligned16({k, v, k_out, vt_out})) return FA_ERR_SHAPE;
+  if (2ll * heads * cdiv(S, fa::kFp8ScaleRows) > 0x7fffffffll) return FA_ERR_SHAPE;
+  fa::QuantArgs a{};
+  a.t[0] = {static_cast<const uint16_t*>(k), static_cast<uint8_t*>(k_out), k_scale, 0};
+  a.t[1] = {static_cast<const uint16_t*>(v), static_cast<uint8_t*>(vt_out), v_scale, 1};
+  a.count = 2;
+  a.heads = heads;
+  a.S = S;
+  a.D = D;
+  a.ld = cdiv(S, fa::kFp8ScaleRows) * fa::kFp8ScaleRows;
   return fa::launch_quant_fp8(a, static_cast<hipStream_t>(stream));
 }
 

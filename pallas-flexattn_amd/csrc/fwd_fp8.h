@@ -36,7 +36,7 @@ constexpr int kFp8ScaleRows = 128;  // rows per scale block (queries or keys)
 
 struct Fp8FwdArgs {
   Problem p;
-  const uint8_t* q;      // (B, Hq, Sq, D) e4m3
+  const uint8_t* q;      // (B, Hq, Sq, D) e4m3, or with kQ16 bf16 (q_scale unused)
   const uint8_t* k;      // (B, Hkv, Skv, D) e4m3
   const uint8_t* vt;     // (B, Hkv, D, ldv) e4m3: V transposed, keys padded to ldv
   int ldv;               // multiple of 128, >= Skv; padding keys are zero
@@ -79,7 +79,49 @@ __device__ __forceinline__ f32x16 mma_f8(i32x8 a, i32x8 b, f32x16 acc, int sa, i
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, 0, 0, 0, sa, 0, sb);
 }
 
-template <int D, int NW, bool kMods>
+// Exponent e of a block's scale 2^e: the smallest with 448 2^e >= amax
+// (frexp-style on the ratio, exact), clamped to [-126, 127]: the scale stays a
+// normal float, whose exponent field is its E8M0 code; 0 for an all-zero block
+// or a non-finite amax.
+__device__ __forceinline__ int fp8_scale_exp(float amax) {
+  int e = 0;
+  if (amax > 0.f && amax < INFINITY) {
+    int ex;
+    const float f = frexpf(amax / 448.0f, &ex);  // amax / 448 = f 2^ex, f in [0.5, 1)
+    e = (f == 0.5f) ? ex - 1 : ex;
+    e = e < -126 ? -126 : (e > 127 ? 127 : e);
+  }
+  return e;
+}
+// eight bf16 values times inv as e4m3 (lo: values 0-3, hi: 4-7)
+__device__ __forceinline__ u32x2 fp8_pack8(u32x4 v, float inv) {
+  float x[8];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    x[2 * t] = __uint_as_float(v[t] << 16) * inv;
+    x[2 * t + 1] = __uint_as_float(v[t] & 0xffff0000u) * inv;
+  }
+  int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
+  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], w0, true);
+  int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(x[4], x[5], 0, false);
+  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(x[6], x[7], w1, true);
+  return u32x2{(uint32_t)w0, (uint32_t)w1};
+}
+__device__ __forceinline__ float amax8(u32x4 v, float m) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    m = fmaxf(m, fmaxf(fabsf(__uint_as_float(v[t] << 16)), fabsf(__uint_as_float(v[t] & 0xffff0000u))));
+  return m;
+}
+
+// kQ16: Q arrives in bf16 and is quantised here: a workgroup's 128 rows are
+// one scale block, read by nobody else, so the block maximum takes one pass
+// over registers and the first tile's barrier, and the operand is the bits
+// that quant_fp8_kernel would have written.  Forward from bf16 tensors, Q
+// quantised by a launch of its own / here, K and V in two launches / one:
+// B4 H32 S8192 D128 causal 1468 / 1431 us, B2 H16 S2624 D128 causal 93 / 85,
+// B3 H8 S734 D128 41 / 29.
+template <int D, int NW, bool kMods, bool kQ16 = false>
 // (three waves per SIMD: the 32 KiB of LDS allows five workgroups per CU, and
 // the third wave hides more of the softmax than the registers it takes cost:
 // 8 % faster than two at causal S = 8192; with score mods two, whose 256
@@ -100,6 +142,8 @@ void fwd_fp8_kernel(Fp8FwdArgs a) {
   static_assert(4 * TILE >= BM * 2 * D, "O rows staged through the K / V buffers");
 
   __shared__ __attribute__((aligned(1024))) char lds[4 * TILE];  // K0 K1 V0 V1
+  [[maybe_unused]] __shared__ float qmax[kQ16 ? NW : 1];
+  static_assert(!kQ16 || BM == kFp8ScaleRows, "a workgroup's rows are one scale block");
 
   const Problem& P = a.p;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -113,7 +157,6 @@ void fwd_fp8_kernel(Fp8FwdArgs a) {
   const int qw = q0 + 32 * w + lr;
   const bool qvalid = qw < P.Sq;
   const int skv = P.Skv;
-  const int nqb = (P.Sq + kFp8ScaleRows - 1) / kFp8ScaleRows;
   const int nkb = (skv + kFp8ScaleRows - 1) / kFp8ScaleRows;
   const int kvh = b * P.Hkv + hk;
 
@@ -122,13 +165,22 @@ void fwd_fp8_kernel(Fp8FwdArgs a) {
 
   // Q rows as B operands (rows past the sequence read as zero) and their scale
   i32x8 qf[KS];
-  {
+  int scq = 0;
+  u32x4 qb[kQ16 ? 4 * KS : 1];  // the lane's bf16 row pieces: values 64 s + 32 hh + 8 x ..
+  if constexpr (kQ16) {
+    const i32x4 rq = make_rsrc(reinterpret_cast<const char*>(a.q) + (size_t)head * P.Sq * D * 2, (uint32_t)P.Sq * D * 2);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) qb[4 * s + x] = buf_load16(rq, (qw * D + 64 * s + 32 * hh + 8 * x) * 2);
+  } else {
     const i32x4 rq = make_rsrc(reinterpret_cast<const char*>(a.q) + (size_t)head * P.Sq * D, (uint32_t)P.Sq * D);
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       qf[s] = cat8(buf_load16(rq, qw * D + 64 * s + 32 * hh), buf_load16(rq, qw * D + 64 * s + 32 * hh + 16));
+    const int nqb = (P.Sq + kFp8ScaleRows - 1) / kFp8ScaleRows;
+    scq = e8m0_code(a.q_scale[(size_t)head * nqb + (qvalid ? qw : P.Sq - 1) / kFp8ScaleRows]);
   }
-  const int scq = e8m0_code(a.q_scale[(size_t)head * nqb + (qvalid ? qw : P.Sq - 1) / kFp8ScaleRows]);
   const float slope = P.alibi ? P.alibi[h] : 0.f;
   const float cap_inv = P.softcap > 0.f ? 1.0f / P.softcap : 0.f;
   int klo, khi;
@@ -282,7 +334,31 @@ void fwd_fp8_kernel(Fp8FwdArgs a) {
   auto kbase_of = [&](int it) { return tab.kbase(walk, it, sub_log2, lane); };
   if (n_it > 0) issue(kbase_of(0), 0);
   wait_vmem();
+  if constexpr (kQ16) {
+    float am = 0.f;
+#pragma unroll
+    for (int x = 0; x < 4 * KS; ++x) am = amax8(qb[x], am);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o));
+    if (lane == 0) qmax[w] = am;
+  }
   __syncthreads();
+  if constexpr (kQ16) {
+    float am = qmax[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) am = fmaxf(am, qmax[i]);
+    const int e = fp8_scale_exp(am);
+    const float inv = ldexpf(1.0f, -e);
+    scq = e + 127;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const u32x2 c = fp8_pack8(qb[4 * s + x], inv);
+        qf[s][2 * x] = (int)c[0];
+        qf[s][2 * x + 1] = (int)c[1];
+      }
+  }
   auto tile_step = [&](int it, auto buf_c) {
     constexpr int buf = decltype(buf_c)::value;
     const int kbase = kbase_of(it);
@@ -389,14 +465,20 @@ void fwd_fp8_kernel(Fp8FwdArgs a) {
 // block; the largest power of two whose product with 448 still covers
 // amax; exponent clamped to [-126, 127]), element = RNE(x / scale): the
 // division by a power of two is exact, so the element stays within +-448.
-// One workgroup (256 threads) per block.
+// One workgroup (256 threads) per block; a launch may hold two tensors of one
+// shape (K and V: blocks past the first tensor's belong to the second).
 // With `transpose` the block is written as D rows of the padded key axis
 // (ld bytes per row, V^T layout of the fp8 forward), else row-major.
-struct QuantArgs {
+struct QuantTensor {
   const uint16_t* x;  // (heads, S, D) bf16
   uint8_t* out;       // (heads, S, D) or (heads, D, ld)
   float* scale;       // (heads, ceil(S / 128))
-  int heads, S, D, ld, transpose;
+  int transpose;
+};
+struct QuantArgs {
+  QuantTensor t[2];
+  int count;  // tensors
+  int heads, S, D, ld;
 };
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
@@ -428,12 +510,15 @@ __global__ __launch_bounds__(256) void quant_fp8_kernel(QuantArgs a) {
   static_assert(R == 128 && NT <= 256 && NT == 16 * NCH, "block shape");
   __shared__ float red[4];
   const int nb = (a.S + R - 1) / R;
-  const int head = blockIdx.x / nb, blk = blockIdx.x - head * nb;
+  const int second = blockIdx.x >= (unsigned)(a.heads * nb) ? 1 : 0;
+  const QuantTensor& T = a.t[second];
+  const int bid = blockIdx.x - second * a.heads * nb;
+  const int head = bid / nb, blk = bid - head * nb;
   const int r0 = blk * R;
   const int rows = min(R, a.S - r0);
-  const uint16_t* src = a.x + ((size_t)head * a.S + r0) * D;
+  const uint16_t* src = T.x + ((size_t)head * a.S + r0) * D;
   const int tid = threadIdx.x;
-  const bool tr = a.transpose != 0;
+  const bool tr = T.transpose != 0;
   const bool act = tid < NT;
   const int g = tid & 15, c = tid >> 4;
   auto row_of = [&](int j) { return tr ? 8 * g + j : (tid + NT * j) / NCH; };
@@ -447,53 +532,30 @@ __global__ __launch_bounds__(256) void quant_fp8_kernel(QuantArgs a) {
     if (act && r < rows) v[j] = *reinterpret_cast<const u32x4*>(src + r * D + chunk_of(j) * 8);
   }
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      amax = fmaxf(amax, fabsf(__uint_as_float(v[j][t] << 16)));
-      amax = fmaxf(amax, fabsf(__uint_as_float(v[j][t] & 0xffff0000u)));
-    }
+  for (int j = 0; j < 8; ++j) amax = amax8(v[j], amax);
   // block maximum: across the wave, then the four waves
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  // smallest e with 448 * 2^e >= amax (frexp-style on the ratio, exact)
-  // (clamped to [-126, 127]: the scale stays a normal float, whose exponent
-  // field is its E8M0 code; a non-finite amax leaves scale 1)
-  int e = 0;
-  if (amax > 0.f && amax < INFINITY) {
-    int ex;
-    const float f = frexpf(amax / 448.0f, &ex);  // amax / 448 = f 2^ex, f in [0.5, 1)
-    e = (f == 0.5f) ? ex - 1 : ex;
-    e = e < -126 ? -126 : (e > 127 ? 127 : e);
-  }
+  const int e = fp8_scale_exp(amax);
   const float inv = ldexpf(1.0f, -e);
-  if (tid == 0) a.scale[(size_t)head * nb + blk] = ldexpf(1.0f, e);
+  if (tid == 0) T.scale[(size_t)head * nb + blk] = ldexpf(1.0f, e);
   if (!act) return;
   // convert (rows past S are zero): lo = values 0-3 of the chunk, hi = 4-7
   uint32_t lo[8], hi[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    float x[8];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      x[2 * t] = __uint_as_float(v[j][t] << 16) * inv;
-      x[2 * t + 1] = __uint_as_float(v[j][t] & 0xffff0000u) * inv;
-    }
-    int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
-    w0 = __builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], w0, true);
-    int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(x[4], x[5], 0, false);
-    w1 = __builtin_amdgcn_cvt_pk_fp8_f32(x[6], x[7], w1, true);
-    lo[j] = (uint32_t)w0;
-    hi[j] = (uint32_t)w1;
+    const u32x2 p = fp8_pack8(v[j], inv);
+    lo[j] = p[0];
+    hi[j] = p[1];
   }
   if (!tr) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int r = row_of(j);
-      if (r < rows) *reinterpret_cast<u32x2*>(a.out + ((size_t)head * a.S + r0 + r) * D + chunk_of(j) * 8) = u32x2{lo[j], hi[j]};
+      if (r < rows) *reinterpret_cast<u32x2*>(T.out + ((size_t)head * a.S + r0 + r) * D + chunk_of(j) * 8) = u32x2{lo[j], hi[j]};
     }
     return;
   }
@@ -503,7 +565,7 @@ __global__ __launch_bounds__(256) void quant_fp8_kernel(QuantArgs a) {
   transpose_bytes4(lo[4], lo[5], lo[6], lo[7], th);
   transpose_bytes4(hi[0], hi[1], hi[2], hi[3], tl + 4);
   transpose_bytes4(hi[4], hi[5], hi[6], hi[7], th + 4);
-  uint8_t* dst = a.out + ((size_t)head * D + 8 * c) * a.ld + r0 + 8 * g;
+  uint8_t* dst = T.out + ((size_t)head * D + 8 * c) * a.ld + r0 + 8 * g;
 #pragma unroll
   for (int k = 0; k < 8; ++k) *reinterpret_cast<u32x2*>(dst + (size_t)k * a.ld) = u32x2{tl[k], th[k]};
 }

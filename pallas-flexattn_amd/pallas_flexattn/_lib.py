@@ -72,7 +72,7 @@ class FaFp8Inputs(ctypes.Structure):
                 ("q_scale", _pf), ("k_scale", _pf), ("v_scale", _pf)]
 
 
-EXPORTED = ("fa_fwd", "fa_fwd_fp8", "fa_quantize_fp8", "fa_fwd_host", "fa_bwd_preprocess_host", "fa_bwd_dkdv_host",
+EXPORTED = ("fa_fwd", "fa_fwd_fp8", "fa_fwd_fp8_q16", "fa_quantize_fp8", "fa_quantize_fp8_kv", "fa_fwd_host", "fa_bwd_preprocess_host", "fa_bwd_dkdv_host",
             "fa_bwd_dq_host", "fa_bwd_host", "fa_fwd_splitkv", "fa_fwd_splitkv_workspace_bytes", "fa_fwd_kvcache",
             "fa_fwd_kvcache_workspace_bytes", "fa_bwd", "fa_bwd_workspace_bytes",
             "fa_bwd_noalloc", "fa_bwd_noalloc_max_rows", "fa_bwd_preprocess", "fa_bwd_dkdv", "fa_bwd_dq",
@@ -120,9 +120,13 @@ def load():
         getattr(lib, n).restype = ci
     lib.fa_fwd_fp8.argtypes = [P, ctypes.POINTER(FaFp8Inputs), v, v, v]
     lib.fa_fwd_fp8.restype = ctypes.c_int
+    lib.fa_fwd_fp8_q16.argtypes = lib.fa_fwd_fp8.argtypes
+    lib.fa_fwd_fp8_q16.restype = ctypes.c_int
     i32 = ctypes.c_int32
     lib.fa_quantize_fp8.argtypes = [v, i32, i32, i32, i32, v, v, v]
     lib.fa_quantize_fp8.restype = ctypes.c_int
+    lib.fa_quantize_fp8_kv.argtypes = [v, v, i32, i32, i32, v, v, v, v, v]
+    lib.fa_quantize_fp8_kv.restype = ctypes.c_int
     lib.fa_fwd_kvcache_workspace_bytes.argtypes = [P, KV, ctypes.c_int]
     lib.fa_fwd_kvcache_workspace_bytes.restype = ctypes.c_size_t
     lib.fa_bwd.argtypes = [P, v, v, v, v, v, v, v, v, v, v, ctypes.c_size_t, v]

@@ -42,20 +42,43 @@ def quantize_fp8(x, transpose: bool = False) -> Fp8Tensor:
     """bf16 ``(B, H, S, D)`` GPU tensor -> :class:`Fp8Tensor`: per 128-row
     block scale = 2^e, e the smallest integer with 448 * 2^e >= max |x| of
     the block, elements RNE(x / scale) in e4m3 (``fa_quantize_fp8``)."""
+    x = _bf16_input(x)
+    B, H, S, D = x.shape
+    out, scale = _fp8_empty(x, transpose)
+    _lib.check(_lib.load().fa_quantize_fp8(x.data_ptr(), B * H, S, D, int(transpose), out.data_ptr(),
+                                           scale.data_ptr(), _stream()))
+    scale._fa_scales_ok = scale._version  # powers of two in range by construction
+    return Fp8Tensor(out, scale, S, bool(transpose))
+
+
+def _bf16_input(x):
     import torch
     if x.dim() != 4 or not x.is_cuda or x.dtype != torch.bfloat16:
         raise ValueError("quantize_fp8 takes a bf16 (B, H, S, D) GPU tensor")
-    x = x.contiguous()
+    return x.contiguous()
+
+
+def _fp8_empty(x, transpose):
+    """(codes, scales) buffers of x's quantised form."""
+    import torch
     B, H, S, D = x.shape
     nb = (S + SCALE_ROWS - 1) // SCALE_ROWS
-    ld = nb * SCALE_ROWS
-    out = torch.empty((B, H, D, ld) if transpose else (B, H, S, D), device=x.device, dtype=torch.uint8)
-    scale = torch.empty((B, H, nb), device=x.device, dtype=torch.float32)
-    lib = _lib.load()
-    _lib.check(lib.fa_quantize_fp8(x.data_ptr(), B * H, S, D, int(transpose), out.data_ptr(), scale.data_ptr(),
-                                   _stream()))
-    scale._fa_scales_ok = scale._version  # powers of two in range by construction
-    return Fp8Tensor(out, scale, S, bool(transpose))
+    out = torch.empty((B, H, D, nb * SCALE_ROWS) if transpose else (B, H, S, D), device=x.device, dtype=torch.uint8)
+    return out, torch.empty((B, H, nb), device=x.device, dtype=torch.float32)
+
+
+def _quantize_kv(k, v):
+    """quantize_fp8(k), quantize_fp8(v, transpose=True): one launch for K and V of one shape."""
+    k, v = _bf16_input(k), _bf16_input(v)
+    if k.shape != v.shape or k.device != v.device:
+        return quantize_fp8(k), quantize_fp8(v, transpose=True)
+    B, H, S, D = k.shape
+    (ko, ks), (vo, vs) = _fp8_empty(k, False), _fp8_empty(v, True)
+    _lib.check(_lib.load().fa_quantize_fp8_kv(k.data_ptr(), v.data_ptr(), B * H, S, D, ko.data_ptr(), ks.data_ptr(),
+                                              vo.data_ptr(), vs.data_ptr(), _stream()))
+    for sc in (ks, vs):
+        sc._fa_scales_ok = sc._version
+    return Fp8Tensor(ko, ks, S, False), Fp8Tensor(vo, vs, S, True)
 
 
 def _check_scales(t: Fp8Tensor, name: str) -> None:
@@ -94,7 +117,7 @@ def flex_attention_fp8(query, key, value, score_mod=None, block_mask: Optional[B
     or a transposed :class:`Fp8Tensor`.  Masks, block tables and score mods
     as :func:`flex_attention` (built-in descriptors; document labels as
     contiguous runs).  Returns bf16 O (and float32 LSE)."""
-    r = Fp8Runner(query, key, value, score_mod, block_mask, scale, enable_gqa)
+    r = Fp8Runner(query, key, value, score_mod, block_mask, scale, enable_gqa, keep_q16=True)
     r.fwd()
     return (r.o, r.lse) if return_lse else r.o
 
@@ -103,41 +126,56 @@ class Fp8Runner:
     """One fp8 forward problem bound to its inputs and outputs: the plan,
     the fa_fp8_inputs struct and O / LSE are built once; ``fwd()`` only
     enqueues the kernel on the current stream (as ``flash_attn.Runner`` does
-    for the bf16 path; used by the benchmark)."""
+    for the bf16 path; used by the benchmark).  bf16 inputs are quantised here,
+    once; with ``keep_q16`` the queries stay bf16 and every ``fwd()`` quantises
+    them in the kernel (the one-shot :func:`flex_attention_fp8`)."""
 
     def __init__(self, query, key, value, score_mod=None, block_mask: Optional[BlockMask] = None,
-                 scale: Optional[float] = None, enable_gqa: bool = False):
+                 scale: Optional[float] = None, enable_gqa: bool = False, keep_q16: bool = False):
         import torch
         from .flash_attn import _get_plan, _resolve, _ShapeOnly, _tables_for
-        q8, k8, v8, mask, score, dims = _prepare(query, key, value, score_mod, block_mask, enable_gqa, _resolve)
+        q, k8, v8, mask, score, dims = _prepare(query, key, value, score_mod, block_mask, enable_gqa, _resolve,
+                                                    keep_q16)
         B, Hq, Sq, D, Hkv, Skv = dims
-        dev = q8.data.device
+        self.q16 = not isinstance(q, Fp8Tensor)  # bf16 queries, quantised by the forward itself
+        dev = q.device if self.q16 else q.data.device
         f8 = torch.float8_e4m3fn
         qs, ks = _ShapeOnly((B, Hq, Sq, D), dev, f8), _ShapeOnly((B, Hkv, Skv, D), dev, f8)
         block_mask, tiles = _tables_for(mask, None, block_mask, qs, ks, DEFAULT_TILES["fp8"])
         self.plan = _get_plan(qs, ks, mask, score, scale, block_mask, tiles)
-        self.inputs = (q8, k8, v8, block_mask)  # kept alive with the struct's pointers
+        self.inputs = (q, k8, v8, block_mask)  # kept alive with the struct's pointers
         self.o = torch.empty((B, Hq, Sq, D), device=dev, dtype=torch.bfloat16)
         self.lse = torch.empty((B, Hq, Sq), device=dev, dtype=torch.float32)
-        self.args = _lib.FaFp8Inputs(q8.data.data_ptr(), k8.data.data_ptr(), v8.data.data_ptr(), v8.data.shape[3],
-                                     q8.scale.data_ptr(), k8.scale.data_ptr(), v8.scale.data_ptr())
-        self.lib = _lib.load()
+        self.args = _lib.FaFp8Inputs(q.data_ptr() if self.q16 else q.data.data_ptr(), k8.data.data_ptr(),
+                                     v8.data.data_ptr(), v8.data.shape[3], None if self.q16 else q.scale.data_ptr(),
+                                     k8.scale.data_ptr(), v8.scale.data_ptr())
+        lib = _lib.load()
+        self.launch = lib.fa_fwd_fp8_q16 if self.q16 else lib.fa_fwd_fp8
 
     def fwd(self):
-        _lib.check(self.lib.fa_fwd_fp8(self.plan.ptr(), _lib.ctypes.byref(self.args), self.o.data_ptr(),
-                                       self.lse.data_ptr(), _stream()))
+        _lib.check(self.launch(self.plan.ptr(), _lib.ctypes.byref(self.args), self.o.data_ptr(),
+                               self.lse.data_ptr(), _stream()))
 
 
-def _prepare(query, key, value, score_mod, block_mask, enable_gqa, resolve):
-    """Quantised inputs (bf16 tensors are quantised here), the resolved mask /
-    score descriptors and the dims (B, Hq, Sq, D, Hkv, Skv), validated."""
+def _prepare(query, key, value, score_mod, block_mask, enable_gqa, resolve, keep_q16):
+    """Quantised inputs (bf16 tensors are quantised here; with ``keep_q16`` the
+    queries stay bf16 for the forward to quantise), the resolved mask / score
+    descriptors and the dims (B, Hq, Sq, D, Hkv, Skv), validated."""
     import torch
-    q8 = query if isinstance(query, Fp8Tensor) else quantize_fp8(query)
-    k8 = key if isinstance(key, Fp8Tensor) else quantize_fp8(key)
-    v8 = value if isinstance(value, Fp8Tensor) else quantize_fp8(value, transpose=True)
-    if q8.transposed or k8.transposed or not v8.transposed:
+    if isinstance(query, Fp8Tensor):
+        q = query
+    else:
+        q = _bf16_input(query)
+        if not keep_q16 or q.shape[2] * q.shape[3] * 2 > 0xffffffff:  # (a head's rows: one 32-bit buffer range)
+            q = quantize_fp8(q)
+    if isinstance(key, Fp8Tensor) or isinstance(value, Fp8Tensor):
+        k8 = key if isinstance(key, Fp8Tensor) else quantize_fp8(key)
+        v8 = value if isinstance(value, Fp8Tensor) else quantize_fp8(value, transpose=True)
+    else:
+        k8, v8 = _quantize_kv(key, value)
+    if (isinstance(q, Fp8Tensor) and q.transposed) or k8.transposed or not v8.transposed:
         raise ValueError("query / key row-major, value transposed (quantize_fp8(v, transpose=True))")
-    B, Hq, Sq, D = q8.shape
+    B, Hq, Sq, D = q.shape
     _, Hkv, Skv, Dk = k8.shape
     if v8.shape != k8.shape or Dk != D or k8.shape[0] != B:
         raise ValueError("query / key / value shapes do not match")
@@ -151,8 +189,10 @@ def _prepare(query, key, value, score_mod, block_mask, enable_gqa, resolve):
     mask, score, mods = resolve(mask_mod, score_mod)
     if mods is not None:
         raise NotImplementedError("the fp8 forward takes the built-in mask / score descriptors")
-    for t, name in ((q8, "query"), (k8, "key"), (v8, "value")):
+    for t, name in ((q, "query"), (k8, "key"), (v8, "value")):
+        if not isinstance(t, Fp8Tensor):
+            continue
         if not (t.data.is_contiguous() and t.scale.is_contiguous() and t.scale.dtype == torch.float32):
             raise ValueError("Fp8Tensor data and scales must be contiguous, scales float32")
         _check_scales(t, name)
-    return q8, k8, v8, mask, score, (B, Hq, Sq, D, Hkv, Skv)
+    return q, k8, v8, mask, score, (B, Hq, Sq, D, Hkv, Skv)

@@ -191,3 +191,23 @@ def test_fp8_scales_must_be_powers_of_two():
     sc[0, 0, 0] = 4.0  # fixed in place: checked again, accepted
     pf.flex_attention_fp8(q8, kb, v8)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,mods", [(1, 2, 2, 1, 64, False), (1, 2, 1, 127, 128, False), (2, 2, 2, 128, 64, True),
+                                               (1, 4, 2, 129, 128, True), (1, 2, 2, 700, 64, False)])
+def test_queries_quantised_in_the_kernel(B, Hq, Hkv, S, D, mods):
+    """bf16 queries (quantised by the forward) and K, V quantised in one launch give bit for bit the
+    results of tensors quantised one by one: ragged blocks, a zero block, blocks of very different size."""
+    import torch
+    import pallas_flexattn as pf
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(B, h, S, D, device="cuda", generator=g).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    q[0, 0, :min(S, 128)] *= 3e-4
+    q[0, 1, :min(S, 128)] = 0
+    k[0, -1] *= 37.0
+    sm = pf.compose_score_mods(pf.alibi_score_mod(Hq), pf.softcap_score_mod(20.0)) if mods else None
+    bm = pf.create_block_mask(pf.causal_mask, B, Hq, S, S, 128)
+    got = pf.flex_attention_fp8(q, k, v, score_mod=sm, block_mask=bm, enable_gqa=Hq != Hkv, return_lse=True)
+    want = pf.flex_attention_fp8(pf.quantize_fp8(q), pf.quantize_fp8(k), pf.quantize_fp8(v, transpose=True), score_mod=sm,
+                                 block_mask=bm, enable_gqa=Hq != Hkv, return_lse=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
