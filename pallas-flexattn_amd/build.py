@@ -20,6 +20,9 @@ UNITS = [(os.path.join(CSRC, "capi.hip"), [], "capi"), (os.path.join(CSRC, "kern
      f"kernels_d{d}_{'bwd' if bwd else 'fwd'}")
     for d in (128, 64, 32) for bwd in (1, 0)]
 SOURCES = sorted({u[0] for u in UNITS})
+# CPython extension over torch tensors (host code, links against torch)
+LAUNCH_SRC = os.path.join(CSRC, "torch_launch.cpp")
+LAUNCH_OUT = os.path.join(HERE, "pallas_flexattn", "_launch.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXX = os.environ.get("CXX", "g++")  # host-only units (.cpp)
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-pthread", "-Wall"]
@@ -108,8 +111,27 @@ def compile_units(extra_flags=(), suffix=".o", out_dir=None, jobs=None):
     return outs, [e for _, e in results]
 
 
+def build_launch() -> str:
+    """pallas_flexattn/_launch.so against the installed torch's headers and libraries."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    lib = os.path.join(root, "lib")
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"]]
+    tmp = LAUNCH_OUT + ".tmp"
+    rc, errs = _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                     *[f"-isystem{d}" for d in inc], LAUNCH_SRC, "-o", tmp, "-L" + lib, "-ltorch_python", "-ltorch_cpu",
+                     "-lc10", "-Wl,-rpath," + lib])
+    if rc != 0:
+        raise RuntimeError(f"compile failed on {os.path.basename(LAUNCH_SRC)} ({rc}):\n{errs}")
+    os.replace(tmp, LAUNCH_OUT)
+    return LAUNCH_OUT
+
+
 def build(verbose: bool = False) -> str:
     tmp = OUT + ".tmp"
+    launch = ThreadPoolExecutor(max_workers=1).submit(build_launch)
     write_rtc_sources()
     objs, logs = compile_units(["-c"])
     rc, errs = _run([HIPCC, "-shared", "-fPIC", "-pthread", *objs, "-o", tmp, "-L/opt/rocm/lib", "-lhiprtc",
@@ -121,6 +143,7 @@ def build(verbose: bool = False) -> str:
             if e.strip():
                 print(e, file=sys.stderr)
     os.replace(tmp, OUT)
+    launch.result()
     return OUT
 
 

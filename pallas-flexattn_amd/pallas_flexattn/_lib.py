@@ -83,6 +83,7 @@ EXPORTED = ("fa_fwd", "fa_fwd_fp8", "fa_fwd_fp8_q16", "fa_quantize_fp8", "fa_qua
 MODS_MASK, MODS_SCORE, MODS_BUILTIN_SCORE = 1, 2, 4
 
 _lib = None
+_launch = None
 
 
 class FlexAttnError(RuntimeError):
@@ -182,6 +183,23 @@ def check(status: int) -> None:
     if status != 0:
         msg = load().fa_strerror(status).decode()
         raise FlexAttnError(f"flexattn C ABI error {status}: {msg}")
+
+
+def launcher():
+    """The torch launch extension (csrc/torch_launch.cpp), bound to the loaded
+    library (raises if it has not been built)."""
+    global _launch
+    if _launch is None:
+        lib = load()
+        try:
+            import torch  # noqa: F401  (the extension links against torch's libraries)
+            from . import _launch as ext
+        except ImportError as e:
+            raise FlexAttnError("pallas_flexattn/_launch.so is missing or does not load: build the library first "
+                                f"(pallas-flexattn_amd/build.py): {e}") from e
+        ext.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (lib.fa_fwd, lib.fa_bwd, lib.fa_bwd_workspace_bytes)))
+        _launch = ext
+    return _launch
 
 
 # Runs fa_mods_compile in a fresh interpreter.  torch ships its own copies of

@@ -69,6 +69,10 @@ def _check_interpret(interpret, t):
 
 
 def _check_inputs(q, k, v, host=False):
+    qs, ks = q.shape, k.shape
+    if (not host and len(qs) == 4 and len(ks) == 4 and v.shape == ks and q.is_cuda and k.is_cuda and v.is_cuda
+            and q.dtype == k.dtype == v.dtype and ks[0] == qs[0] and ks[3] == qs[3] and ks[1] and qs[1] % ks[1] == 0):
+        return  # the usual call; anything else is told what is wrong below
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be (B, H, T, D)")
     if host:
@@ -148,6 +152,7 @@ class _Plan:
         self.dname = dname
         import ctypes
         self._ref = ctypes.byref(self.params)
+        self.addr = ctypes.addressof(self.params)
 
     def ptr(self):
         return self._ref
@@ -171,6 +176,29 @@ def _get_plan(q, k, mask, score, scale, block_mask, tiles) -> _Plan:
     if len(_PLAN_CACHE) >= _PLAN_CACHE_MAX:
         _PLAN_CACHE.pop(next(iter(_PLAN_CACHE)))
     _PLAN_CACHE[key] = (plan, block_mask)
+    return plan
+
+
+_CALL_CACHE = {}
+
+
+def _call_plan(q, k, mask, score, scale, block_mask, tiles) -> _Plan:
+    """The plan of a call without user mods: :func:`_tables_for` and
+    :func:`_get_plan` behind one lookup (same key, with the caller's block
+    mask, which the entry keeps alive, and tiles)."""
+    key = (q.shape, k.shape, q.dtype, q.device, None if mask is None else mask.key(),
+           None if score is None else score.key(), scale, None if block_mask is None else id(block_mask), tiles)
+    hit = _CALL_CACHE.get(key)
+    if hit is not None and hit[1] is block_mask:
+        return hit[0]
+    bm, t = _tables_for(mask, None, block_mask, q, k, tiles)
+    plan = _get_plan(q, k, mask, score, scale, bm, t)
+    while len(_CALL_CACHE) >= _PLAN_CACHE_MAX:
+        try:
+            _CALL_CACHE.pop(next(iter(_CALL_CACHE)), None)
+        except (StopIteration, RuntimeError):  # another thread changed it meanwhile
+            break
+    _CALL_CACHE[key] = (plan, block_mask)
     return plan
 
 
@@ -396,6 +424,12 @@ def _fwd_core(q, k, v, mask, score, scale, block_mask, tiles, mods=None, host=Fa
         o = torch.zeros_like(q)
         lse = torch.full(q.shape[:3], -math.inf, device=q.device, dtype=torch.float32)
         return o, lse, None
+    if mods is None and not host:
+        plan = _call_plan(q, k, mask, score, scale, block_mask, tuple(tiles))
+        rc, o, lse = _lib.launcher().fwd(plan.addr, q, k, v, _stream())
+        if rc:
+            _lib.check(rc)
+        return o, lse, plan
     q, k, v = _dense16(q), _dense16(k), _dense16(v)
     if mods is not None:
         tiles = _MODS_TILES[_dtype_code(q)[1]]
@@ -407,8 +441,6 @@ def _fwd_core(q, k, v, mask, score, scale, block_mask, tiles, mods=None, host=Fa
     ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr())
     if host:
         _lib.check(lib.fa_fwd_host(plan.ptr(), *ptrs, 0))
-    elif mods is None:
-        _lib.check(lib.fa_fwd(plan.ptr(), *ptrs, _stream()))
     else:
         h, bufs, n = _mods_args(mods, plan, q, score)
         _lib.check(lib.fa_mods_fwd(h, plan.ptr(), bufs, n, *ptrs, _stream()))
@@ -425,6 +457,13 @@ def _bwd_core(q, k, v, o, lse, do, mask, score, scale, block_mask, tiles, mods=N
         _host_mods(mods)
     if q.numel() == 0 or k.shape[2] == 0:  # no (query, key) pair: zero gradients
         return torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    if mods is None and not host:
+        if plan is None:
+            plan = _call_plan(q, k, mask, score, scale, block_mask, tuple(tiles))
+        rc, dq, dk, dv = _lib.launcher().bwd(plan.addr, q, k, v, o, lse, do, _stream())
+        if rc:
+            _lib.check(rc)
+        return dq, dk, dv
     if do.dtype != q.dtype:
         do = do.to(q.dtype)
     q, k, v, o, do = (_dense16(t) for t in (q, k, v, o, do))
@@ -450,11 +489,8 @@ def _bwd_core(q, k, v, o, lse, do, mask, score, scale, block_mask, tiles, mods=N
     dv = torch.empty_like(v)
     ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), do.data_ptr(), dq.data_ptr(),
             dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws.numel())
-    if mods is None:
-        _lib.check(lib.fa_bwd(plan.ptr(), *ptrs, _stream()))
-    else:
-        h, bufs, n = _mods_args(mods, plan, q, score)
-        _lib.check(lib.fa_mods_bwd(h, plan.ptr(), bufs, n, *ptrs, _stream()))
+    h, bufs, n = _mods_args(mods, plan, q, score)
+    _lib.check(lib.fa_mods_bwd(h, plan.ptr(), bufs, n, *ptrs, _stream()))
     return dq, dk, dv
 
 
@@ -691,6 +727,7 @@ class _FlexFn:
                 @staticmethod
                 def forward(ctx, q, k, v, cfg):
                     # cfg: mask, score, scale, block mask, tiles, mods, host
+                    ctx.set_materialize_grads(False)  # no zeros for the LSE's absent gradient (a launch)
                     o, lse, plan = _fwd_core(q, k, v, *cfg)
                     ctx.save_for_backward(q, k, v, o, lse)
                     ctx.cfg = cfg
@@ -701,6 +738,8 @@ class _FlexFn:
                 @staticmethod
                 def backward(ctx, do, dlse):
                     q, k, v, o, lse = ctx.saved_tensors
+                    if do is None:
+                        do = torch.zeros_like(o)
                     dq, dk, dv = _bwd_core(q, k, v, o, lse, do, *ctx.cfg, plan=ctx.plan)
                     return dq, dk, dv, None
 
@@ -755,7 +794,9 @@ def flex_decode(query, key, value, score_mod: Optional[ScoreSpec] = None, block_
         if k.dim() != 4 or k.shape != v.shape:
             raise ValueError("paged key / value caches must be (num_pages, Hkv, page_size, D)")
         num_pages, Hkv, page_size, D = k.shape
-        pt = page_table.to(device=q.device, dtype=torch.int32).contiguous()
+        pt = page_table
+        if pt.dtype != torch.int32 or pt.device != q.device or not pt.is_contiguous():
+            pt = pt.to(device=q.device, dtype=torch.int32).contiguous()
         if pt.dim() != 2 or pt.shape[0] != q.shape[0]:
             raise ValueError("page_table must be (B, max_pages)")
         Skv = int(kv_len) if kv_len is not None else pt.shape[1] * page_size
@@ -782,7 +823,10 @@ def flex_decode(query, key, value, score_mod: Optional[ScoreSpec] = None, block_
         kvc = _lib.FaKvCache()
         keep = []
         if kv_lens is not None:
-            kl = torch.as_tensor(kv_lens, device=q.device).to(torch.int32).contiguous()
+            kl = kv_lens
+            if not (isinstance(kl, torch.Tensor) and kl.dtype == torch.int32 and kl.device == q.device
+                    and kl.is_contiguous()):
+                kl = torch.as_tensor(kl, device=q.device).to(torch.int32).contiguous()
             if kl.shape != (q.shape[0],):
                 raise ValueError("kv_lens must have one entry per batch row")
             keep.append(kl)

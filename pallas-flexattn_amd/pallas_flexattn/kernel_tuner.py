@@ -256,6 +256,20 @@ def tuned_tiles(seq_len: int, head_dim: int, dtype: str, sparse) -> Optional[Tup
     the shape (the closest measured class: a block-sparse lower triangle)."""
     cls = _class_of(sparse)
     table = load_tune_table()
+    hit = _TILES.get((seq_len, head_dim, dtype, cls))
+    if hit is not None and hit[0] is table:  # (a changed file is another table)
+        return hit[1]
+    tiles = _lookup_tiles(table, seq_len, head_dim, dtype, cls)
+    if len(_TILES) > 256:
+        _TILES.clear()
+    _TILES[(seq_len, head_dim, dtype, cls)] = (table, tiles)
+    return tiles
+
+
+_TILES: Dict[tuple, tuple] = {}
+
+
+def _lookup_tiles(table, seq_len: int, head_dim: int, dtype: str, cls: str):
     e = table.get(table_key(seq_len, head_dim, dtype, cls))
     if e is None and cls in ("window", "document"):
         e = table.get(table_key(seq_len, head_dim, dtype, "causal"))

@@ -277,3 +277,61 @@ def test_empty_problems_launch_nothing():
     torch.cuda.synchronize()
     assert not o.any() and bool(torch.isneginf(lse).all())
     assert not q.grad.any() and kv.grad.shape == kv.shape
+
+
+@pytest.mark.parametrize("form", ["strided", "misaligned", "do-fp32", "expanded-do", "hooks"])
+def test_operand_forms_of_the_native_launch(form):
+    """Operands the launch has to make dense or convert give the dense call's results bit for bit."""
+    import torch
+    import pallas_flexattn as pf
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v, do = (torch.randn(1, 2, 130, 64, device="cuda", generator=g).to(torch.bfloat16) for _ in range(4))
+    if form == "expanded-do":
+        do = do[:, :, :1, :1].expand(1, 2, 130, 64)
+
+    def run(q, k, v, do):
+        t = [x.detach().requires_grad_() for x in (q, k, v)]
+        o = pf.flash_attention(*t, mask_mod=pf.causal_mask)
+        return (o.detach(),) + torch.autograd.grad(o, t, do)
+
+    want = run(q, k, v, do.contiguous())
+    if form == "strided":
+        q, k, do = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, do))
+    elif form == "misaligned":
+        def shift(x):
+            flat = torch.empty(x.numel() + 1, device="cuda", dtype=x.dtype)[1:]
+            return flat.copy_(x.reshape(-1)).view(x.shape)
+        q, v, do = shift(q), shift(v), shift(do)
+        assert q.data_ptr() % 16
+    elif form == "do-fp32":
+        do = do.float()
+    if form == "hooks":
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda()):
+            got = run(q, k, v, do)
+    elif form == "do-fp32":
+        t = [x.detach().requires_grad_() for x in (q, k, v)]
+        o = pf.flash_attention(*t, mask_mod=pf.causal_mask)
+        lse = pf.flash_attention_fwd(q, k, v, mask_mod=pf.causal_mask)[1]
+        assert lse.dtype == torch.bfloat16  # the reference's LSE dtype, converted by the backward
+        got = (o.detach(),) + pf.flash_attention_bwd(q, k, v, o.detach(), _fp32_lse(q, k, v), do, mask_mod=pf.causal_mask)
+    else:
+        got = run(q, k, v, do)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _fp32_lse(q, k, v):
+    import pallas_flexattn as pf
+    bm = pf.create_block_mask(pf.causal_mask, 1, 2, 130, 130, 128)
+    return pf.flex_attention(q, k, v, block_mask=bm, return_lse=True)[1]
+
+
+def test_native_launch_refuses_mismatched_backward_operands():
+    import torch
+    import pallas_flexattn as pf
+    q = torch.randn(1, 2, 64, 64, device="cuda").to(torch.bfloat16)
+    o, lse = pf.flash_attention_fwd(q, q, q)
+    for bad in (dict(o=o[:, :, :32]), dict(do=o[:, :1]), dict(logsumexp=lse[:, :, :1]), dict(do=o.cpu())):
+        args = dict(q=q, k=q, v=q, o=o, logsumexp=lse, do=o, **{})
+        args.update(bad)
+        with pytest.raises(ValueError):
+            pf.flash_attention_bwd(**args)
