@@ -286,15 +286,22 @@ void dq_bf16_kernel(BwdArgs a) {
         }
       }
       if constexpr (kMasked) {
-        // key kbase + 32 j + acc_row(e, hh), compared against tile-relative
-        // bounds (a constant per element)
-        const int lo = klo - kbase - 32 * j - 8 * hh, hi = khi - kbase - 32 * j - 8 * hh;
+        // element e: key base + acc_row(e, 0); nothing to drop where every row of
+        // the wave sees the whole sub-tile (as in the forward)
+        const int base = kbase + 32 * j + 8 * hh;
+        if (Mod::kMask || !__all(!qvalid || (klo <= kbase + 32 * j && khi >= kbase + 32 * j + 31))) {
+          uint32_t bits = interval_bits(klo - base, khi - base);
+          if constexpr (Mod::kMask) {
+            uint32_t user = 0u;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int c = acc_row(e, 0);
-          bool keep = c >= lo && c <= hi;
-          if constexpr (Mod::kMask) keep = keep && Mod::mask(P, b, h, qw, kbase + 32 * j + c + 8 * hh);
-          sacc[e] = keep ? sacc[e] : -INFINITY;
+            for (int e = 0; e < 16; ++e) {
+              const int r = acc_row(e, 0);
+              user |= Mod::mask(P, b, h, qw, base + r) ? (1u << r) : 0u;
+            }
+            bits &= user;
+          }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sacc[e] = keep_bit(sacc[e], bits, acc_row(e, 0), -INFINITY);
         }
       }
 #pragma unroll
@@ -610,10 +617,7 @@ __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
 #pragma unroll
       for (int j = 0; j < NQS; ++j) {
         const int base = qbase + 32 * j + 8 * hh;
-        const int lo = max(qlo - base, 0), hi = min(qhi - base, 31);
-        const uint32_t up = 0xffffffffu >> (31 - max(hi, 0));
-        const uint32_t dn = 0xffffffffu << min(lo, 31);
-        rmask[j] = (hi >= lo) ? (up & dn) : 0u;
+        rmask[j] = interval_bits(qlo - base, qhi - base);
         if constexpr (Mod::kMask) {  // user mask on the rows this lane holds
           uint32_t bits = 0u;
 #pragma unroll

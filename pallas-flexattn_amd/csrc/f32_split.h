@@ -395,13 +395,21 @@ __device__ __forceinline__ bool fwd_split_item(const FwdArgs& a, char* lds, uint
     }
     if (masked) {
       if (em.interval) {
-        const int lo = em.lo - kbase - 8 * hh, hi = em.hi - kbase - 8 * hh;
+        // (nothing to drop where every row of the wave sees the whole tile)
+        if (Mod::kMask || !__all(!qvalid || (em.lo <= kbase && em.hi >= kbase + 31))) {
+          const int base = kbase + 8 * hh;
+          uint32_t bits = interval_bits(em.lo - base, em.hi - base);
+          if constexpr (Mod::kMask) {
+            uint32_t user = 0u;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int c = acc_row(e, 0);
-          bool keep = c >= lo && c <= hi;
-          if constexpr (Mod::kMask) keep = keep && Mod::mask(P, b, h, qw, kbase + c + 8 * hh);
-          sacc[e] = keep ? sacc[e] : -INFINITY;
+            for (int e = 0; e < 16; ++e) {
+              const int r = acc_row(e, 0);
+              user |= Mod::mask(P, b, h, qw, base + r) ? (1u << r) : 0u;
+            }
+            bits &= user;
+          }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sacc[e] = keep_bit(sacc[e], bits, acc_row(e, 0), -INFINITY);
         }
       } else {
 #pragma unroll
@@ -605,14 +613,24 @@ __device__ __forceinline__ bool dq_split_item(const BwdArgs& a, char* lds, uint3
     }
     if (masked) {
       if (em.interval) {
-        const int lo = em.lo - kbase - 8 * hh, hi = em.hi - kbase - 8 * hh;
+        // (nothing to drop where every row of the wave sees the whole tile)
+        if (Mod::kMask || !__all(!qvalid || (em.lo <= kbase && em.hi >= kbase + 31))) {
+          const int base = kbase + 8 * hh;
+          uint32_t bits = interval_bits(em.lo - base, em.hi - base);
+          if constexpr (Mod::kMask) {
+            uint32_t user = 0u;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int c = acc_row(e, 0);
-          bool keep = c >= lo && c <= hi;
-          if constexpr (Mod::kMask) keep = keep && Mod::mask(P, b, h, qw, kbase + c + 8 * hh);
-          sacc[e] = keep ? sacc[e] : -INFINITY;
-          if constexpr (kMods) dsdx[e] = keep ? dsdx[e] : 0.f;
+            for (int e = 0; e < 16; ++e) {
+              const int r = acc_row(e, 0);
+              user |= Mod::mask(P, b, h, qw, base + r) ? (1u << r) : 0u;
+            }
+            bits &= user;
+          }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            sacc[e] = keep_bit(sacc[e], bits, acc_row(e, 0), -INFINITY);
+            if constexpr (kMods) dsdx[e] = keep_bit(dsdx[e], bits, acc_row(e, 0), 0.f);
+          }
         }
       } else {
 #pragma unroll
@@ -830,14 +848,24 @@ __device__ __forceinline__ bool dkdv_split_item(const BwdArgs& a, char* lds, flo
     }
     if (masked) {
       if (em.interval) {
-        const int lo = em.lo - qbase - 8 * hh, hi = em.hi - qbase - 8 * hh;
+        // (nothing to drop where every row of the wave sees the whole tile)
+        if (Mod::kMask || !__all(!kvalid || (em.lo <= qbase && em.hi >= qbase + 31))) {
+          const int base = qbase + 8 * hh;
+          uint32_t bits = interval_bits(em.lo - base, em.hi - base);
+          if constexpr (Mod::kMask) {
+            uint32_t user = 0u;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int c = acc_row(e, 0);
-          bool keep = c >= lo && c <= hi;
-          if constexpr (Mod::kMask) keep = keep && Mod::mask(P, b, hq, qbase + c + 8 * hh, kw);
-          sacc[e] = keep ? sacc[e] : -INFINITY;
-          if constexpr (kMods) dsdx[e] = keep ? dsdx[e] : 0.f;
+            for (int e = 0; e < 16; ++e) {
+              const int r = acc_row(e, 0);
+              user |= Mod::mask(P, b, hq, base + r, kw) ? (1u << r) : 0u;
+            }
+            bits &= user;
+          }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            sacc[e] = keep_bit(sacc[e], bits, acc_row(e, 0), -INFINITY);
+            if constexpr (kMods) dsdx[e] = keep_bit(dsdx[e], bits, acc_row(e, 0), 0.f);
+          }
         }
       } else {
 #pragma unroll

@@ -414,20 +414,29 @@ void fwd_bf16_kernel(FwdArgs a) {
                                              &dsdx);
           }
       }
-      if (masked) {  // partial tile: keys outside [klo, khi] are dropped
+      // partial tile: keys outside [klo, khi] are dropped, unless every row of
+      // this wave sees all of the tile (rows past Sq see what they like): of a
+      // causal block's diagonal that is a quarter of the tiles, and every tile of
+      // a ragged last query block, which the tables list as partial
+      if (masked && (Mod::kMask || !__all(!qvalid || (klo <= kbase && khi >= kbase + BN - 1)))) {
         const float dead = rform ? INFINITY : -INFINITY;  // the y whose logit is -inf
-        // key kbase + c_e with c_e = 32 j + acc_row(e, hh): the bounds are
-        // taken relative to the tile, so each element compares a constant
-        const int lo = klo - kbase - 8 * hh, hi = khi - kbase - 8 * hh;
 #pragma unroll
-        for (int j = 0; j < NSUB; ++j)
+        for (int j = 0; j < NSUB; ++j) {
+          // element e of sub-tile j: key base + r, r = acc_row(e, 0) < 24
+          const int base = kbase + 32 * j + 8 * hh;
+          uint32_t bits = interval_bits(klo - base, khi - base);
+          if constexpr (Mod::kMask) {
+            uint32_t user = 0u;
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int c = 32 * j + acc_row(e, 0);
-            bool keep = c >= lo && c <= hi;
-            if constexpr (Mod::kMask) keep = keep && Mod::mask(P, b, h, qw, kbase + c + 8 * hh);
-            sacc[j][e] = keep ? sacc[j][e] : dead;
+            for (int e = 0; e < 16; ++e) {
+              const int r = acc_row(e, 0);
+              user |= Mod::mask(P, b, h, qw, base + r) ? (1u << r) : 0u;
+            }
+            bits &= user;
           }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sacc[j][e] = keep_bit(sacc[j][e], bits, acc_row(e, 0), dead);
+        }
       }
       // V^T fragments of d tile i (two tiles in flight): tile 0's reads issue
       // before the softmax, tile i + 1's before tile i's MFMAs

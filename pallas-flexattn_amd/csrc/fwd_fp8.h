@@ -417,16 +417,17 @@ void fwd_fp8_kernel(Fp8FwdArgs a) {
           }
         }
       }
-      if (masked) {  // partial tile: keys outside [klo, khi] are dropped
+      // partial tile: keys outside [klo, khi] are dropped, unless every row of
+      // this wave sees all of the tile (as in the bf16 forward)
+      if (masked && !__all(!qvalid || (klo <= kbase && khi >= kbase + BN - 1))) {
         const float dead = rform ? INFINITY : -INFINITY;  // the y whose logit is -inf
-        const int lo = klo - kbase - 16 * hh, hi = khi - kbase - 16 * hh;  // tile-relative bounds
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+          const int base = kbase + 32 * j + 16 * hh;
+          const uint32_t bits = interval_bits(klo - base, khi - base);
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int c = 32 * j + e;
-            sacc[j][e] = (c >= lo && c <= hi) ? sacc[j][e] : dead;
-          }
+          for (int e = 0; e < 16; ++e) sacc[j][e] = keep_bit(sacc[j][e], bits, e, dead);
+        }
       }
       i32x8 pf;
       softmax(sacc, pf);

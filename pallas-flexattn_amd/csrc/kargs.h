@@ -118,6 +118,24 @@ __device__ __forceinline__ bool mod_keep(const Problem& P, int b, int h, int q, 
   else return k >= lo && k <= hi;
 }
 
+// Bits [max(lo, 0), min(hi, 31)] of a 32-position block (none when empty):
+// the positions of a partial tile that an interval mask keeps, one bit test per
+// element.  Compared element by element instead, the 16 to 32 conditions of a
+// tile live in SGPR pairs and spill: a partial tile of the forward then took
+// twice a full one's time (causal S3000 H8 D128: 104 us; S2944 58).
+__device__ __forceinline__ uint32_t interval_bits(int lo, int hi) {
+  lo = lo > 0 ? lo : 0;
+  hi = hi < 31 ? hi : 31;
+  const uint32_t up = 0xffffffffu >> (31 - (hi > 0 ? hi : 0));
+  const uint32_t dn = 0xffffffffu << (lo < 31 ? lo : 31);
+  return hi >= lo ? (up & dn) : 0u;
+}
+// x where bit r of bits is set, else dead
+__device__ __forceinline__ float keep_bit(float x, uint32_t bits, int r, float dead) {
+  const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)bits, r, 1);
+  return __uint_as_float((__float_as_uint(x) & m) | (__float_as_uint(dead) & ~m));
+}
+
 // mask_ok under the policy (generic kernels).
 template <class Mod>
 __device__ __forceinline__ bool mod_mask_ok(const Problem& P, int b, int h, int q, int k, int qdoc, int kdoc) {
