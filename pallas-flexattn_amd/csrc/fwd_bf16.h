@@ -333,12 +333,20 @@ void fwd_bf16_kernel(FwdArgs a) {
     const bool more = it + AHEAD < it1;
     Copy nc;
     if (more) nc = issue_plan(kbase_of(it + AHEAD), (buf + AHEAD) % NS);
-    if (NS > 1 && kbase >= skv && more) {
+    masked = masked || (kbase + BN > skv);
+    // a partial tile that no row of this wave sees (two of the eight wave tiles
+    // of a diagonal block) only issues its copies: forward at D = 128, causal
+    // S8192 2018 -> 1986 us, S2048 160 -> 157, window 1024 648 -> 631; at D = 64
+    // the test costs what it saves (and in dQ its registers: 209 -> 236 us, spills)
+    bool run = kbase < skv;
+    if constexpr (D == 128 && NS > 1 && !Mod::kMask) {  // (NS = 1 has a barrier inside)
+      if (masked) run = run && __any(qvalid && klo <= kbase + BN - 1 && khi >= kbase);
+    }
+    if (NS > 1 && !run && more) {
 #pragma unroll
       for (int i = 0; i < 2 * IPW; ++i) issue_one(nc, i);
     }
-    if (kbase < skv) {  // workgroup-uniform
-      masked = masked || (kbase + BN > skv);
+    if (run) {  // wave-uniform
       const char* kl = lds + buf * TILE;
       const char* vl = lds + (NS + buf) * TILE;
 
