@@ -81,14 +81,18 @@ inline int default_tiles(const fa_params* p, Tiles* t) {
 // The dK/dV query tile of a bf16 backward.  128 rows (four 32-row sub-tiles,
 // half the tile boundaries of 64) run with the interval-mask kernel, D >= 64,
 // 128-key workgroups and q-side tables at a multiple of 128 rows; the
-// automatic choice takes them for D = 128 (step 9.10-9.14 against 9.33-9.36 ms
-// at causal B4 H32 S8192 D128) and 64 rows otherwise (D = 64: the 64-row tile
-// is 6 % faster at causal B4 H32 S4096, tuner measurement).  A requested tile
-// (fa_params.block_q) that the call cannot run is refused.
+// automatic choice takes them at D = 128 (step 9.10-9.14 against 9.33-9.36 ms
+// at causal B4 H32 S8192 D128) and at D = 64 without score mods (dK/dV, 64 /
+// 128 rows: causal B4 H32 S4096 561 / 532 us, B4 H16 S2048 83 / 79, B4 Hq16 Hkv4
+// S2048 164 / 136, B2 H8 S1000 24 / 22, dense B1 Hq8 Hkv4 S3059 116 / 100;
+// with a soft-cap the larger tile's 264 registers leave one wave per SIMD:
+// B4 H16 S2048 115 / 133).  A requested tile (fa_params.block_q) that the call
+// cannot run is refused.
 inline int dkdv_query_tile(const fa_params* p, const Problem& pr, Tiles* t) {
   if (p->dtype != FA_DTYPE_BF16) return FA_OK;  // fp32: 32 (default_tiles)
   const bool q128 = p->D >= 64 && t->bkv == 128 && interval_masks(pr) && (!pr.has_tables || pr.mblk_q % 128 == 0);
-  if (t->bq == 0) t->bq = (q128 && p->D >= 128) ? 128 : 64;
+  const bool mods = pr.alibi != nullptr || pr.softcap > 0.f;
+  if (t->bq == 0) t->bq = (q128 && (p->D >= 128 || !mods)) ? 128 : 64;
   return (t->bq == 128 && !q128) ? FA_ERR_UNSUPPORTED : FA_OK;
 }
 

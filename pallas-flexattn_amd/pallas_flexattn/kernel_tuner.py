@@ -95,7 +95,7 @@ def print_kernel_config(
     config = get_kernel_config(batch_size, num_heads, seq_len, head_dim, mask_type)
     cls = {"causal": "causal", "sliding_window": "window", "document": "document"}.get(mask_type, "dense")
     bm, bn, bkv, bq, ns = resolved_tiles(kernel_tiles(config['block_r'], config['block_c'], "bf16", seq_len,
-                                                      head_dim, cls), "bf16", head_dim)
+                                                      head_dim, cls), "bf16", head_dim, score_mods=False)
     print("=" * 70)
     print("MI355X FlexAttention Kernel Configuration")
     print("=" * 70)
@@ -146,13 +146,14 @@ def full_tiles(tiles, dtype: str) -> Tuple[int, int, int, int, int]:
     return t + DEFAULT_TILES[dtype][len(t):]
 
 
-def resolved_tiles(tiles, dtype: str, head_dim: int) -> Tuple[int, int, int, int, int]:
+def resolved_tiles(tiles, dtype: str, head_dim: int, score_mods: bool = True) -> Tuple[int, int, int, int, int]:
     """The tiles a call runs (automatic entries made explicit): BLOCK_Q 128
-    for bf16 with D = 128 and BLOCK_KV 128 (the C ABI's choice under window /
-    document masks and 128-row tables), else 64 (fp32: 32); 2 LDS stages."""
+    for bf16 with BLOCK_KV 128 at D = 128, and at D = 64 where the call has no
+    score mods (the C ABI's choice under window / document masks and 128-row
+    tables), else 64 (fp32: 32); 2 LDS stages."""
     bm, bn, bkv, bq, ns = full_tiles(tiles, dtype)
     if not bq:
-        bq = (128 if head_dim >= 128 and bkv == 128 else 64) if dtype == "bf16" else 32
+        bq = (128 if head_dim >= (128 if score_mods else 64) and bkv == 128 else 64) if dtype == "bf16" else 32
     return bm, bn, bkv, bq, ns or 2
 
 

@@ -136,3 +136,33 @@ def test_tiles_reach_the_c_abi():
     b = pf.flex_attention(q, q, q, block_mask=bm)
     torch.cuda.synchronize()
     assert float((a.float() - b.float()).abs().max()) < 2e-2
+
+
+@pytest.mark.parametrize("mods", [False, True], ids=["plain", "mods"])
+@pytest.mark.parametrize("kind,Hq,Hkv,S", [("causal", 4, 4, 129), ("causal", 8, 2, 383), ("window", 4, 2, 257),
+                                           ("none", 4, 2, 31), ("none", 2, 2, 640)])
+def test_dkdv_query_tile_rule_d64(kind, Hq, Hkv, S, mods):
+    """D = 64, no tile asked for: dK / dV are those of the 128-query tile, or
+    with score mods of the 64-query tile (bit for bit), and the oracle's."""
+    import torch
+    import pallas_flexattn as pf
+    print(f"[gpu tiles] dkdv rule {kind} {Hq} {Hkv} {S} {mods}", flush=True)
+    q, k, v, do = inputs(7, 1, Hq, Hkv, S, S, 64, "bf16")
+    omask = oracle_mask(kind, S, S, 1, 100, 20) if kind == "window" else oracle_mask(kind, S, S)
+    mm = {"causal": pf.causal_mask, "window": pf.sliding_window_mask(100, 20), "none": None}[kind]
+    bm = pf.create_block_mask(mm, 1, Hq, S, S, 128) if mm is not None else None
+    score = pf.softcap_score_mod(20.0) if mods else None
+
+    def grads(opts):
+        t = [to_torch(x, "bf16").requires_grad_() for x in (q, k, v)]
+        o = pf.flex_attention(*t, score_mod=score, block_mask=bm, enable_gqa=Hq != Hkv, kernel_options=opts)
+        o.backward(to_torch(do, "bf16"))
+        return t[1].grad, t[2].grad
+
+    auto = grads({"BLOCK_M": 128})  # a key of its own, so no tuned entry decides BLOCK_Q
+    same = grads({"BLOCK_M": 128, "BLOCK_KV": 128, "BLOCK_Q": 64 if mods else 128})
+    torch.cuda.synchronize()
+    _, _, (_, wdk, wdv) = oracle_fwd_bwd(q, k, v, do, omask, softcap=20.0 if mods else None)
+    for nm, got, want, s in (("dK", auto[0], wdk, same[0]), ("dV", auto[1], wdv, same[1])):
+        assert_close(f"{kind} {nm}", to_np(got), want, BF16_TOL)
+        assert torch.equal(got, s)
