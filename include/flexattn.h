@@ -229,6 +229,17 @@ int fa_bwd(const fa_params *p, const void *q, const void *k, const void *v, cons
            const float *lse, const void *dout, void *dq, void *dk, void *dv, void *workspace,
            size_t workspace_bytes, void *stream);
 
+/* fa_bwd where the dK/dV of a bf16 GQA problem with few work items may be split
+ * over the q heads of each group, as its size and mask suggest: fp32 partial
+ * sums in the workspace (at most 64 MiB beside Delta) and a third launch that
+ * adds them in a fixed order - fa_bwd's sums in another order.  Other problems,
+ * and a workspace of fa_bwd_workspace_bytes(p) bytes or one that is not 16-byte
+ * aligned, run as fa_bwd.  No reference counterpart. */
+size_t fa_bwd_split_workspace_bytes(const fa_params *p);
+int fa_bwd_split(const fa_params *p, const void *q, const void *k, const void *v, const void *o,
+                 const float *lse, const void *dout, void *dq, void *dk, void *dv, void *workspace,
+                 size_t workspace_bytes, void *stream);
+
 /* fa_bwd without a workspace, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No reference counterpart: the reference's XLA runtime always

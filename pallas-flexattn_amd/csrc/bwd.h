@@ -37,6 +37,10 @@ struct BwdArgs {
   // bf16 dQ tile kernel only: compute Delta itself from O and dO and write it
   // to `delta` (the whole backward then runs dQ before dK/dV, no Delta pass)
   int fuse_delta;
+  // bf16 dK/dV over `parts` runs of a GQA group's q heads (dkdv_bf16_kernel's
+  // kParts form): fp32 partial sums, part (parts, items, 2, waves, D * 32)
+  float* part;
+  int parts;
 };
 
 // sum_j O[j] dO[j] over one 16-byte chunk of bf16 (8 elements), in the order

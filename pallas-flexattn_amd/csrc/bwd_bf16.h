@@ -430,7 +430,10 @@ void dq_bf16_kernel(BwdArgs a) {
 }
 
 // ---------------------------------------------------------------- dK dV ----
-template <int D, int BQ, int NW, bool kMods, class Mod = BuiltinMod>
+// kParts: a work item takes one of a.parts runs of the GQA group's q heads and
+// leaves its dK / dV sums in a.part as fp32, in register order (1 KiB stores);
+// dkdv_merge_kernel adds the runs up in a fixed order and rounds once.
+template <int D, int BQ, int NW, bool kMods, class Mod = BuiltinMod, bool kParts = false>
 __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
   using E = Elt<uint16_t>;
   using frag = E::frag;
@@ -450,10 +453,20 @@ __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 31, hh = lane >> 5;
   const int nkt = (P.Skv + BKV - 1) / BKV;
-  const int g = P.Hq / P.Hkv;
-  int head, kt;
-  work_item(blockIdx.x, P.B * P.Hkv, nkt, P.xcd_remap, P.head_group_kv, true, &head, &kt);
+  int g = P.Hq / P.Hkv;
+  int head, kt, part = 0;
+  if constexpr (kParts) {
+    // (the parts of a kv head count as heads; all heads in one group of the XCD order)
+    const int nh = P.B * P.Hkv * a.parts;
+    work_item(blockIdx.x, nh, nkt, P.xcd_remap, nh >> 3, true, &head, &kt);
+    part = head % a.parts;
+    head /= a.parts;
+    g /= a.parts;
+  } else {
+    work_item(blockIdx.x, P.B * P.Hkv, nkt, P.xcd_remap, P.head_group_kv, true, &head, &kt);
+  }
   const int b = head / P.Hkv, hk = head - b * P.Hkv;
+  const int hq0 = kParts ? (hk * a.parts + part) * g : hk * g;
   const int k0 = kt * BKV;
   const int kw = k0 + 32 * w + lr;
   const bool kvalid = kw < P.Skv;
@@ -465,7 +478,7 @@ __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
   const bool spec0 = P.has_tables && (P.tab_h == 1 || g == 1);
   int first_full = 0, first_part = 0;
   if (spec0) {
-    const int row = tab_row(P, b, hk * g, k0 / P.mblk_kv, P.n_kvblk);
+    const int row = tab_row(P, b, hq0, k0 / P.mblk_kv, P.n_kvblk);
     if (P.full_q_num) first_full = vload_i32(P.full_q_idx + (size_t)row * P.q_width, 0, P.q_width);
     if (P.q_num) first_part = vload_i32(P.q_idx + (size_t)row * P.q_width, 0, P.q_width);
   }
@@ -511,7 +524,7 @@ __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
   QWalk walk;
   walk.P = &P;
   walk.b = b;
-  walk.hq0 = hk * g;
+  walk.hq0 = hq0;
   walk.g = g;
   walk.kvrow = k0 / P.mblk_kv;
   walk.sub = P.mblk_q / BQ;
@@ -882,6 +895,19 @@ __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
     mfma_drain<'a'>(dka[i]);
     mfma_drain<'a'>(dva[i]);
   }
+  if constexpr (kParts) {
+    f32x4* out = reinterpret_cast<f32x4*>(a.part) +
+                 (((size_t)part * (P.B * P.Hkv) + head) * nkt + kt) * (2 * NW * D * 8) + w * (D * 8) + lane;
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        out[(4 * i + j) * 64] = f32x4{dka[i][4 * j], dka[i][4 * j + 1], dka[i][4 * j + 2], dka[i][4 * j + 3]};
+        out[NW * (D * 8) + (4 * i + j) * 64] =
+            f32x4{dva[i][4 * j], dva[i][4 * j + 1], dva[i][4 * j + 2], dva[i][4 * j + 3]};
+      }
+    return;
+  }
   // dK, dV rows of this wave, staged through the (now idle) tile buffers
   {
     const int rows_left = P.Skv - (k0 + 32 * w);
@@ -891,6 +917,35 @@ __global__ __launch_bounds__(NW * 64) void dkdv_bf16_kernel(BwdArgs a) {
     store_rows_bf16<D>(dka, P.scale, stage, dkp, rows_left, lane);
     store_rows_bf16<D>(dva, 1.0f, stage + 32 * RB, dvp, rows_left, lane);
   }
+}
+
+// dK / dV from the fp32 sums of a.parts runs of q heads, added in order; the
+// grid is (items, 2): blockIdx.y 0 is dK, 1 is dV.  Each wave takes 32 keys.
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64) void dkdv_merge_kernel(BwdArgs a) {
+  constexpr int DT = D / 32, RB = D * 2;
+  __shared__ __attribute__((aligned(16))) char lds[NW * 32 * RB];
+  const Problem& P = a.p;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int nkt = (P.Skv + 32 * NW - 1) / (32 * NW);
+  const int item = blockIdx.x, head = item / nkt, row0 = (item - head * nkt) * 32 * NW + 32 * w;
+  const f32x4* in = reinterpret_cast<const f32x4*>(a.part) + (size_t)item * (2 * NW * D * 8) +
+                    (blockIdx.y * NW + w) * (D * 8) + lane;
+  const size_t part_stride = (size_t)gridDim.x * (2 * NW * D * 8);
+  f32x16 acc[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i) zero(acc[i]);
+  for (int t = 0; t < a.parts; ++t, in += part_stride)
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 x = in[(4 * i + j) * 64];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[i][4 * j + c] += x[c];
+      }
+  uint16_t* rows = static_cast<uint16_t*>(blockIdx.y ? a.dv : a.dk) + ((size_t)head * P.Skv + row0) * D;
+  store_rows_bf16<D>(acc, blockIdx.y ? 1.0f : P.scale, lds + w * (32 * RB), rows, P.Skv - row0, lane);
 }
 
 }  // namespace fa

@@ -132,7 +132,8 @@ int device_cus() {
 }
 
 // Validates the params for the requested backward stages and launches them.
-int bwd_stages(const fa_params* p, BwdArgs& a, int stages, hipStream_t s) {
+// part_bytes: room at a.part for the partial sums of a split dK/dV (0: none).
+int bwd_stages(const fa_params* p, BwdArgs& a, int stages, hipStream_t s, size_t part_bytes = 0) {
   if (!p) return FA_ERR_NULL;
   (void)device_scratch();
   if (p->dtype == FA_DTYPE_FP8_E4M3) return FA_ERR_DTYPE;  // the fp8 path is forward-only
@@ -150,6 +151,10 @@ int bwd_stages(const fa_params* p, BwdArgs& a, int stages, hipStream_t s) {
     if ((stages & kStageDkdv) && !a.p.q_num && !a.p.full_q_num) return FA_ERR_TABLES;
   }
   t.ng = fa::f32_groups(p, fa::dq_grid(a.p, t.bm), device_cus());
+  if (stages == kStageAll && a.part) {
+    a.parts = fa::dkdv_parts(p, a.p, t, device_cus());
+    if (part_bytes < fa::dkdv_part_bytes(p, a.p, a.parts)) a.parts = 1;
+  }
   const bool m = has_mods(a.p);
   if (p->dtype == FA_DTYPE_BF16)
     return m ? bwd_d<uint16_t, true>(a, p->D, t, stages, s) : bwd_d<uint16_t, false>(a, p->D, t, stages, s);
@@ -378,13 +383,25 @@ size_t fa_bwd_workspace_bytes(const fa_params* p) {
   return delta_bytes(p);
 }
 
-int fa_bwd(const fa_params* p, const void* q, const void* k, const void* v, const void* o,
-           const float* lse, const void* dout, void* dq, void* dk, void* dv, void* workspace,
-           size_t workspace_bytes, void* stream) {
+size_t fa_bwd_split_workspace_bytes(const fa_params* p) {
+  if (!p) return 0;
+  size_t bytes = delta_bytes(p);
+  Tiles t;
+  Problem pr;
+  if (p->dtype == FA_DTYPE_BF16 && default_tiles(p, &t) == FA_OK && build_problem(p, t, &pr) == FA_OK &&
+      dkdv_query_tile(p, pr, &t) == FA_OK)
+    bytes += fa::dkdv_part_bytes(p, pr, fa::dkdv_parts(p, pr, t, device_cus()));
+  return bytes;
+}
+
+static int bwd_launch(const fa_params* p, const void* q, const void* k, const void* v, const void* o,
+                      const float* lse, const void* dout, void* dq, void* dk, void* dv, void* workspace,
+                      size_t workspace_bytes, bool split, void* stream) {
   if (!p) return FA_ERR_NULL;
   if (!q || !k || !v || !o || !lse || !dout || !dq || !dk || !dv) return FA_ERR_NULL;
   if (!aligned16({q, k, v, o, dout, dq, dk, dv})) return FA_ERR_SHAPE;
-  if (!workspace || workspace_bytes < delta_bytes(p)) return FA_ERR_WORKSPACE;
+  const size_t db = delta_bytes(p);
+  if (!workspace || workspace_bytes < db) return FA_ERR_WORKSPACE;
   BwdArgs a{};
   a.q = q;
   a.k = k;
@@ -396,7 +413,20 @@ int fa_bwd(const fa_params* p, const void* q, const void* k, const void* v, cons
   a.dk = dk;
   a.dv = dv;
   a.delta = static_cast<float*>(workspace);
-  return bwd_stages(p, a, kStageAll, static_cast<hipStream_t>(stream));
+  if (split && aligned16({workspace})) a.part = a.delta + db / sizeof(float);
+  return bwd_stages(p, a, kStageAll, static_cast<hipStream_t>(stream), workspace_bytes - db);
+}
+
+int fa_bwd(const fa_params* p, const void* q, const void* k, const void* v, const void* o,
+           const float* lse, const void* dout, void* dq, void* dk, void* dv, void* workspace,
+           size_t workspace_bytes, void* stream) {
+  return bwd_launch(p, q, k, v, o, lse, dout, dq, dk, dv, workspace, workspace_bytes, false, stream);
+}
+
+int fa_bwd_split(const fa_params* p, const void* q, const void* k, const void* v, const void* o,
+                 const float* lse, const void* dout, void* dq, void* dk, void* dv, void* workspace,
+                 size_t workspace_bytes, void* stream) {
+  return bwd_launch(p, q, k, v, o, lse, dout, dq, dk, dv, workspace, workspace_bytes, true, stream);
 }
 
 size_t fa_bwd_noalloc_max_rows(void) { return kScratchFloats; }

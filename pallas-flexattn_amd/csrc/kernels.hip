@@ -124,6 +124,14 @@ template <typename T, int D, int BQ, int NW, bool M>
 int run_dkdv(const BwdArgs& a, hipStream_t s) {
   const int grid = dkdv_grid(a.p, 32 * NW);
   if constexpr (sizeof(T) == 2) {
+    if constexpr (D >= 64 && NW == 4) {
+      if (a.parts > 1) {  // the C ABI: interval masks and a workspace for the partial sums
+        hipLaunchKernelGGL((fa::dkdv_bf16_kernel<D, BQ, NW, M, fa::BuiltinMod, true>), dim3(grid * a.parts),
+                           dim3(NW * 64), 0, s, a);
+        hipLaunchKernelGGL((fa::dkdv_merge_kernel<D, NW>), dim3(grid, 2), dim3(NW * 64), 0, s, a);
+        return launch_status();
+      }
+    }
     if (interval_masks(a.p)) {
       hipLaunchKernelGGL((fa::dkdv_bf16_kernel<D, BQ, NW, M>), dim3(grid), dim3(NW * 64), 0, s, a);
       return launch_status();

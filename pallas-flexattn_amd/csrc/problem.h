@@ -96,6 +96,33 @@ inline int dkdv_query_tile(const fa_params* p, const Problem& pr, Tiles* t) {
   return (t->bq == 128 && !q128) ? FA_ERR_UNSUPPORTED : FA_OK;
 }
 
+// Into how many runs of q heads the dK/dV of a bf16 GQA group is split (1: not
+// at all).  A work item walks the q tiles of all the group's heads, so few kv
+// heads or short keys give fewer items than compute units and each of them is
+// long; the runs' fp32 sums cost a write, a read and a launch.  The largest
+// divisor of the group that leaves at most one round of workgroups (one per
+// compute unit at D = 128, two at D = 64), or two where causal or document
+// walks differ in length and the short ones fill in behind the long.  Measured,
+// whole backward, unsplit / split (us): causal D128 B1 Hq32 Hkv8 S1024
+// 133 / 74, S3000 389 / 290, S4096 585 / 460, B1 Hq32 Hkv1 S1024 767 / 104;
+// causal D64 B4 Hq16 Hkv4 S2048 195 / 150, B8 343 / 290; dense D128 B1 Hq8 Hkv4
+// S4096 300 / 245.  Past the limit: causal D128 B2 Hq32 Hkv8 S4096 880 / 898,
+// window 1024 B1 Hq32 Hkv8 S4096 260 / 276, dense B1 Hq16 Hkv8 S4096 437 / 453.
+// Where the longest item would get fewer than 3 tiles shorter, the second
+// launch costs as much (dense D64 B7 Hq8 Hkv4 S238 21.7 / 23.4).
+inline int dkdv_parts(const fa_params* p, const Problem& pr, const Tiles& t, int cus) {
+  if (p->dtype != FA_DTYPE_BF16 || p->D < 64 || t.bkv != 128 || !interval_masks(pr)) return 1;
+  const int g = pr.Hq / pr.Hkv, nqt = cdiv(pr.Sq, t.bq);
+  const bool equal_walks = !pr.q_doc && (pr.win_left < 0) == (pr.win_right < 0);
+  const long long limit = (long long)cus * (p->D == 64 ? 2 : 1) * (equal_walks ? 1 : 2);
+  for (int d = g; d > 1; --d)
+    if (g % d == 0 && (long long)dkdv_grid(pr, t.bkv) * d <= limit) return (g - g / d) * nqt >= 3 ? d : 1;
+  return 1;
+}
+inline size_t dkdv_part_bytes(const fa_params* p, const Problem& pr, int parts) {
+  return parts > 1 ? (size_t)parts * dkdv_grid(pr, 128) * 2 * 128 * p->D * sizeof(float) : 0;
+}
+
 // float32 forward and dQ: a work item's key tiles are shared by two groups of
 // waves where the grid (`items` workgroups) gives a compute unit at most two
 // workgroups, so that the longest walks take half the steps; larger grids fill

@@ -41,7 +41,7 @@ const at::Tensor* tensor(PyObject* x) {
   return &THPVariable_Unpack(x);
 }
 
-// bind(fa_fwd, fa_bwd, fa_bwd_workspace_bytes)
+// bind(fa_fwd, fa_bwd_split, fa_bwd_split_workspace_bytes)
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3) {
     PyErr_SetString(PyExc_TypeError, "bind takes 3 addresses");

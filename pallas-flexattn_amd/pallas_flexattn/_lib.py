@@ -74,7 +74,8 @@ class FaFp8Inputs(ctypes.Structure):
 
 EXPORTED = ("fa_fwd", "fa_fwd_fp8", "fa_fwd_fp8_q16", "fa_quantize_fp8", "fa_quantize_fp8_kv", "fa_fwd_host", "fa_bwd_preprocess_host", "fa_bwd_dkdv_host",
             "fa_bwd_dq_host", "fa_bwd_host", "fa_fwd_splitkv", "fa_fwd_splitkv_workspace_bytes", "fa_fwd_kvcache",
-            "fa_fwd_kvcache_workspace_bytes", "fa_bwd", "fa_bwd_workspace_bytes",
+            "fa_fwd_kvcache_workspace_bytes", "fa_bwd", "fa_bwd_workspace_bytes", "fa_bwd_split",
+            "fa_bwd_split_workspace_bytes",
             "fa_bwd_noalloc", "fa_bwd_noalloc_max_rows", "fa_bwd_preprocess", "fa_bwd_dkdv", "fa_bwd_dq",
             "fa_mask_build_workspace_bytes", "fa_build_block_mask", "fa_strerror", "fa_abi_version",
             "fa_mods_compile", "fa_mods_free_blob", "fa_mods_load", "fa_mods_unload", "fa_mods_fwd", "fa_mods_bwd",
@@ -130,8 +131,9 @@ def load():
     lib.fa_quantize_fp8_kv.restype = ctypes.c_int
     lib.fa_fwd_kvcache_workspace_bytes.argtypes = [P, KV, ctypes.c_int]
     lib.fa_fwd_kvcache_workspace_bytes.restype = ctypes.c_size_t
-    lib.fa_bwd.argtypes = [P, v, v, v, v, v, v, v, v, v, v, ctypes.c_size_t, v]
-    lib.fa_bwd.restype = ctypes.c_int
+    for f in (lib.fa_bwd, lib.fa_bwd_split):
+        f.argtypes = [P, v, v, v, v, v, v, v, v, v, v, ctypes.c_size_t, v]
+        f.restype = ctypes.c_int
     lib.fa_bwd_noalloc.argtypes = [P, v, v, v, v, v, v, v, v, v, v]
     lib.fa_bwd_noalloc.restype = ctypes.c_int
     lib.fa_bwd_noalloc_max_rows.argtypes = []
@@ -142,8 +144,9 @@ def load():
     lib.fa_bwd_dkdv.restype = ctypes.c_int
     lib.fa_bwd_dq.argtypes = [P, v, v, v, v, v, v, v, v]
     lib.fa_bwd_dq.restype = ctypes.c_int
-    lib.fa_bwd_workspace_bytes.argtypes = [P]
-    lib.fa_bwd_workspace_bytes.restype = ctypes.c_size_t
+    for f in (lib.fa_bwd_workspace_bytes, lib.fa_bwd_split_workspace_bytes):
+        f.argtypes = [P]
+        f.restype = ctypes.c_size_t
     M = ctypes.POINTER(FaMaskBuild)
     lib.fa_mask_build_workspace_bytes.argtypes = [M]
     lib.fa_mask_build_workspace_bytes.restype = ctypes.c_size_t
@@ -197,7 +200,8 @@ def launcher():
         except ImportError as e:
             raise FlexAttnError("pallas_flexattn/_launch.so is missing or does not load: build the library first "
                                 f"(pallas-flexattn_amd/build.py): {e}") from e
-        ext.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (lib.fa_fwd, lib.fa_bwd, lib.fa_bwd_workspace_bytes)))
+        ext.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (lib.fa_fwd, lib.fa_bwd_split,
+                                                                            lib.fa_bwd_split_workspace_bytes)))
         _launch = ext
     return _launch
 

@@ -448,7 +448,7 @@ def _fwd_core(q, k, v, mask, score, scale, block_mask, tiles, mods=None, host=Fa
 
 
 def _bwd_core(q, k, v, o, lse, do, mask, score, scale, block_mask, tiles, mods=None, host=False, plan=None):
-    """Backward through fa_bwd (fa_mods_bwd with user mods; fa_bwd_host on
+    """Backward through fa_bwd_split (fa_mods_bwd with user mods; fa_bwd_host on
     the host path) -> (dq, dk, dv).  ``plan`` is the forward's plan when the
     caller has it (same problem), else one is looked up."""
     torch = _torch()
@@ -632,8 +632,8 @@ class Runner:
         self.delta = torch.empty(q.shape[:3], device=q.device, dtype=torch.float32)
         self.dq, self.dk, self.dv = torch.empty_like(self.q), torch.empty_like(self.k), torch.empty_like(self.v)
         self.lib = _lib.load()
-        # fa_bwd's workspace holds Delta (B, Hq, Sq) fp32
-        self.ws = torch.empty(max(self.lib.fa_bwd_workspace_bytes(self.plan.ptr()), 256), device=q.device,
+        # the workspace holds Delta (B, Hq, Sq) fp32 and a split dK/dV's partial sums
+        self.ws = torch.empty(max(self.lib.fa_bwd_split_workspace_bytes(self.plan.ptr()), 256), device=q.device,
                               dtype=torch.uint8)
 
     def fwd(self):
@@ -655,12 +655,12 @@ class Runner:
                                       self.dq.data_ptr(), _stream()))
 
     def bwd(self):
-        """The whole backward (fa_bwd): for bf16 interval masks the dQ kernel
+        """The whole backward (fa_bwd_split): for bf16 interval masks the dQ kernel
         computes Delta, then dK/dV; otherwise Delta, dK/dV, dQ."""
-        _lib.check(self.lib.fa_bwd(self.plan.ptr(), self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
-                                   self.o.data_ptr(), self.lse.data_ptr(), self.do.data_ptr(), self.dq.data_ptr(),
-                                   self.dk.data_ptr(), self.dv.data_ptr(), self.ws.data_ptr(), self.ws.numel(),
-                                   _stream()))
+        _lib.check(self.lib.fa_bwd_split(self.plan.ptr(), self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
+                                         self.o.data_ptr(), self.lse.data_ptr(), self.do.data_ptr(), self.dq.data_ptr(),
+                                         self.dk.data_ptr(), self.dv.data_ptr(), self.ws.data_ptr(), self.ws.numel(),
+                                         _stream()))
 
     def step(self):
         """One forward + backward pass."""

@@ -355,7 +355,7 @@ static void model_dq(const Problem& P, bool fuse) {
 
 // ---- dK / dV (dkdv_bf16_kernel) --------------------------------------------
 template <int D, int BQ, int NW>
-static void model_dkdv(const Problem& P) {
+static void model_dkdv(const Problem& P, int parts) {
   constexpr int BKV = 32 * NW, RB = D * 2, KSTEPS = D / 16, DT = D / 32, NQS = BQ / 32, TILE = BQ * RB;
   constexpr int IPW = TILE / 1024 / NW, STAT = 1024, NST = BQ / 64;
   constexpr int LDS = 4 * TILE + 4 * STAT;
@@ -379,19 +379,29 @@ static void model_dkdv(const Problem& P) {
           for (int rd = 0; rd < 2; ++rd) inside(rt.tr[rd][dt] + 16 * c * RB, 8, TILE, "dK/dV Q^T / dO^T read");
       inside(w * 2 * 32 * RB, 2 * 32 * RB, LDS, "dK/dV staging");
     }
-  const int g = P.Hq / P.Hkv;
+  const int g = P.Hq / P.Hkv / parts;  // q heads of one part of a GQA group
   const int nkt = (P.Skv + BKV - 1) / BKV;
   const int grid = dkdv_grid(P, BKV);
   const long long q_rows = (long long)P.B * P.Hq * P.Sq, kv_rows = (long long)P.B * P.Hkv * P.Skv;
-  for (int bid = 0; bid < grid; ++bid) {
+  std::vector<char> seen((size_t)grid * parts, 0);
+  for (int bid = 0; bid < grid * parts; ++bid) {
+    const int nh = P.B * P.Hkv * parts;
     int head, kt;
-    work_item(bid, P.B * P.Hkv, nkt, P.xcd_remap, P.head_group_kv, true, &head, &kt);
-    inside(head, 1, P.B * P.Hkv, "dK/dV work item head");
+    work_item(bid, nh, nkt, P.xcd_remap, parts > 1 ? nh >> 3 : P.head_group_kv, true, &head, &kt);
+    inside(head, 1, nh, "dK/dV work item head");
+    inside(kt, 1, nkt, "dK/dV work item key tile");
+    const int part = head % parts;
+    head /= parts;
     const int b = head / P.Hkv, hk = head - b * P.Hkv;
+    const int hq0 = (hk * parts + part) * g;
+    // every part of every item once, its partial sums in a slot of its own
+    const long long slot = ((long long)part * (P.B * P.Hkv) + head) * nkt + kt;
+    inside(slot, 1, (long long)grid * parts, "dK/dV partial sums");
+    if (seen[slot]++) fail("a part of a dK/dV item runs twice");
     const int k0 = kt * BKV;
     // the first tile's entries, requested before the counts
     if (P.has_tables && (P.tab_h == 1 || g == 1)) {
-      const int row = tab_row(P, b, hk * g, k0 / P.mblk_kv, P.n_kvblk);
+      const int row = tab_row(P, b, hq0, k0 / P.mblk_kv, P.n_kvblk);
       if (P.full_q_num) HostLoad::vector(P.full_q_idx + (long long)row * P.q_width, 0, P.q_width);
       if (P.q_num) HostLoad::vector(P.q_idx + (long long)row * P.q_width, 0, P.q_width);
     }
@@ -407,7 +417,7 @@ static void model_dkdv(const Problem& P) {
     QWalkT<HostLoad> walk;
     walk.P = &P;
     walk.b = b;
-    walk.hq0 = hk * g;
+    walk.hq0 = hq0;
     walk.g = g;
     walk.kvrow = k0 / P.mblk_kv;
     walk.sub = P.mblk_q / BQ;
@@ -448,20 +458,20 @@ static void run_fwd(const Problem& P, const Tiles& t, const FwdOpts& o) {
 }
 
 template <int D>
-static void run_bwd(const Problem& P, const Tiles& t) {
+static void run_bwd(const Problem& P, const Tiles& t, int parts) {
   if constexpr (D >= 64) {
     if (t.bn == 32) model_dq<D, 32, 4>(P, true);
     else if (t.bn == 128) model_dq<D, 128, 4>(P, true);
     else if (t.bm == 256) model_dq<D, 64, 8>(P, true);
     else if (t.bm == 64) model_dq<D, 64, 2>(P, true);
     else model_dq<D, 64, 4>(P, true);
-    if (t.bkv == 64) return model_dkdv<D, 64, 2>(P);
-    if (t.bq == 128) return model_dkdv<D, 128, 4>(P);
+    if (t.bkv == 64) return model_dkdv<D, 64, 2>(P, 1);
+    if (t.bq == 128) return model_dkdv<D, 128, 4>(P, parts);
   } else {
     if (t.bm == 64) model_dq<D, 64, 2>(P, true);
     else model_dq<D, 64, 4>(P, true);
   }
-  model_dkdv<D, 64, 4>(P);
+  model_dkdv<D, 64, 4>(P, parts);
 }
 
 static const int kTileSets[][5] = {  // bm, bn, bkv, bq, stages (0: automatic)
@@ -505,7 +515,9 @@ static int check_case(Case& c) {
     if (dkdv_query_tile(&p, P, &t) != FA_OK) continue;
     if (P.has_tables && (P.mblk_kv % t.bkv || P.mblk_q % t.bq)) continue;
     g_where = "backward";
-    if (c.D == 32) run_bwd<32>(P, t); else if (c.D == 64) run_bwd<64>(P, t); else run_bwd<128>(P, t);
+    const int parts = dkdv_parts(&p, P, t, 256);
+    if (dkdv_part_bytes(&p, P, parts) > (64u << 20)) fail("partial sums of dK/dV above 64 MiB");
+    if (c.D == 32) run_bwd<32>(P, t, parts); else if (c.D == 64) run_bwd<64>(P, t, parts); else run_bwd<128>(P, t, parts);
     ++launches;
   }
   return launches;

@@ -166,3 +166,49 @@ def test_dkdv_query_tile_rule_d64(kind, Hq, Hkv, S, mods):
     for nm, got, want, s in (("dK", auto[0], wdk, same[0]), ("dV", auto[1], wdv, same[1])):
         assert_close(f"{kind} {nm}", to_np(got), want, BF16_TOL)
         assert torch.equal(got, s)
+
+
+@pytest.mark.parametrize("kind,B,Hq,Hkv,S,D,mods", [
+    ("causal", 1, 8, 1, 200, 128, False), ("causal", 1, 6, 2, 129, 64, False), ("doc", 2, 8, 2, 320, 64, False),
+    ("window", 1, 12, 4, 383, 128, False), ("none", 3, 8, 2, 257, 64, True), ("causal", 2, 16, 4, 130, 128, True)])
+def test_dkdv_split_over_q_heads(kind, B, Hq, Hkv, S, D, mods):
+    """GQA with few work items: dK / dV from the runs of q heads, against the
+    oracle, and against the unsplit kernel (a workspace with room for Delta
+    only, and one at 4 bytes past a 16-byte boundary)."""
+    import torch
+    import pallas_flexattn as pf
+    from pallas_flexattn.flash_attn import Runner
+    print(f"[gpu tiles] dkdv split {kind} {B} {Hq} {Hkv} {S} {D} {mods}", flush=True)
+    q, k, v, do = inputs(11, B, Hq, Hkv, S, S, D, "bf16")
+    mm, omask, score, cap = None, oracle_mask("none", S, S), None, None
+    if kind == "doc":
+        dm = pf.document_mask([[S // 3, S - S // 3]] * B)
+        mm, omask = pf.and_masks(dm, pf.causal_mask), oracle_mask("causal", S, S, B, doc_ids=dm.doc_ids)
+    elif kind == "window":
+        mm, omask = pf.sliding_window_mask(100, 20), oracle_mask("window", S, S, 1, 100, 20)
+    elif kind == "causal":
+        mm, omask = pf.causal_mask, oracle_mask("causal", S, S)
+    if mods:
+        score, cap = pf.softcap_score_mod(20.0), 20.0
+    r = Runner(*(to_torch(x, "bf16") for x in (q, k, v, do)), mask_mod=mm, score_mod=score)
+    delta = (B * Hq * S * 4 + 255) & ~255
+    assert r.ws.numel() > delta  # the call is one that splits
+    r.step()
+    split = r.dk.clone(), r.dv.clone()
+    r.step()
+    assert torch.equal(split[0], r.dk) and torch.equal(split[1], r.dv)  # a fixed order of sums
+    ws = r.ws
+    whole = []
+    for w in (ws[:delta], torch.empty(ws.numel() + 16, device="cuda", dtype=torch.uint8)[4:]):
+        r.ws = w
+        r.bwd()
+        whole.append((r.dk.clone(), r.dv.clone()))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(*whole))
+    _, _, (_, wdk, wdv) = oracle_fwd_bwd(q, k, v, do, omask, softcap=cap)
+    for nm, got, one, want in (("dK", split[0], whole[0][0], wdk), ("dV", split[1], whole[0][1], wdv)):
+        assert_close(f"{kind} {nm}", to_np(got), want, BF16_TOL)
+        # the same fp32 products in another order, each rounded once: at most
+        # one bf16 step (2^-7 of the value), and fp32 rounding of the sums
+        d = (got.float() - one.float()).abs()
+        assert bool((d <= one.float().abs() * 2.0 ** -7 + one.float().abs().max() * 2.0 ** -16).all())
