@@ -14,9 +14,9 @@
 // 32 x 32 x 16 block, the eight v_mfma_f32_32x32x2f32 they replace 512.
 //
 // Times (us; forward, dK/dV, dQ; float32 instructions -> this file):
-//   B4 H8  S1000 D64  causal   150, 190, 163  ->   47, 101,  61
+//   B4 H8  S1000 D64  causal   150, 190, 163  ->   42,  90,  58
 //   B4 H16 S4096 D64  causal  1287, 2982, 1770 -> 732, 1530, 982
-//   B2 H16 S2048 D128 causal   474, 680, 460  ->  255,  448, 277
+//   B2 H16 S2048 D128 causal   474, 680, 460  ->  231,  428, 277
 // Bound by the chain of a tile (products, exponentials, splitting, products):
 // the large shape runs at 178 to 209 TFLOP/s, 1.07 to 1.25 PFLOP/s of bf16
 // products, what the library's bf16 GEMM reaches on this board.

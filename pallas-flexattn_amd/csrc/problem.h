@@ -127,7 +127,8 @@ inline size_t dkdv_part_bytes(const fa_params* p, const Problem& pr, int parts) 
 // waves where the grid (`items` workgroups) gives a compute unit at most two
 // workgroups, so that the longest walks take half the steps; larger grids fill
 // the SIMDs by themselves and keep the tiles in one group (f32_split.h has no
-// room for two groups at D = 128).  Measured, causal D = 64, one group / two:
+// room for two groups at D = 128).  Measured (before partial tiles took their
+// masks as bits, about 10 % off both sides), causal D = 64, one group / two:
 // 256 items (B4 H8 S1000) forward 62 / 47 us, dQ 76 / 61; 512 items 73 / 65
 // and 93 / 86; 1024 items 116 / 127 and 151 / 166; 2048 items (B4 H16 S4096)
 // 732 / 721 and 982 / 1028.
