@@ -450,9 +450,9 @@ def derivative(e: Expr) -> Expr:
         return _add(_mul(derivative(a[0]), a[1]), _mul(a[0], derivative(a[1])))
     if op == "truediv":
         da, db = derivative(a[0]), derivative(a[1])
-        if _is(db, 0.0) or _is(db, 0):  # constant divisor: (u / c)' = u' (1 / c)
+        if _is(db, 0.0) or _is(db, 0):  # a divisor without the score: (u / c)' = u' (1 / c)
             inv = _fconst(1.0 / float(np.float32(a[1].value))) if _is_factor(a[1]) else binop("truediv", ONE, a[1])
-        return _mul(da, inv)
+            return _mul(da, inv)
         num = _add(_mul(da, a[1]), _mul(_fconst(-1), _mul(a[0], db)))
         return binop("truediv", num, binop("mul", a[1], a[1])) if not _is(num, 0.0) else ZERO
     if op == "neg":

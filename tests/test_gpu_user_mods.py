@@ -57,6 +57,10 @@ def _case_mods(name, Hq, S):
             return s - 0.05 * s * s, 1.0 - 0.1 * s
         return (lambda q, kv: (q - kv <= 70) & (kv - q <= 30), lambda b, h, q, k: (q - k <= 70) & (k - q <= 30),
                 lambda s, b, h, q, kv: s - 0.05 * s * s, np_score)
+    if name == "softsign-causal":  # a divisor that depends on the score
+        def np_score(s, b, h, q, k):
+            return 4.0 * s / (1.0 + np.abs(s)), 4.0 / (1.0 + np.abs(s)) ** 2
+        return ("causal", None, lambda s, b, h, q, kv: 4.0 * s / (1.0 + torch.abs(s)), np_score)
     raise ValueError(name)
 
 
@@ -71,6 +75,8 @@ CASES = [
     ("banded-per-head", "bf16", 1, 4, 4, 512, 128),
     ("quadratic-score-window", "fp32", 1, 2, 2, 256, 32),
     ("quadratic-score-window", "bf16", 1, 2, 2, 256, 32),
+    ("softsign-causal", "bf16", 1, 4, 2, 320, 64),
+    ("softsign-causal", "fp32", 1, 2, 2, 200, 64),
 ]
 
 

@@ -67,6 +67,14 @@ SCORES = {
     "quadratic_exp": (lambda s, b, h, q, kv: 0.1 * s * s + torch.exp(s / 8.0) + (q % 3)),
     "clamp_where": (lambda s, b, h, q, kv: torch.where(s > 2.0, 2.0 + 0.5 * (s - 2.0), torch.clamp(s, min=-3.0))),
     "sigmoid_log": (lambda s, b, h, q, kv: torch.log(torch.sigmoid(s) + 1.0) + torch.sqrt(s * s + 1.0)),
+    # quotients: the divisor depends on the score, on the position only, or is a constant
+    "softsign": (lambda s, b, h, q, kv: s / (1.0 + torch.abs(s))),
+    "rational": (lambda s, b, h, q, kv: 3.0 * s / (1.0 + s * s)),
+    "logistic": (lambda s, b, h, q, kv: 1.0 / (1.0 + torch.exp(-s))),
+    "algebraic": (lambda s, b, h, q, kv: s / torch.sqrt(1.0 + s * s)),
+    "reciprocal": (lambda s, b, h, q, kv: 5.0 / (20.0 + s)),
+    "by_position": (lambda s, b, h, q, kv: s / (1 + torch.abs(q - kv))),
+    "by_constant": (lambda s, b, h, q, kv: (s * s + s) / 3.7),
 }
 
 
