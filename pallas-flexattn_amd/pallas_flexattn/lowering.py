@@ -410,18 +410,30 @@ def _add(a, b):
     return binop("add", a, b)
 
 
+def _f32(v) -> float:
+    """v rounded to float32, the precision of the generated literals."""
+    with np.errstate(over="ignore", under="ignore"):
+        return float(np.float32(v))
+
+
+def _is_normal(v) -> bool:
+    """Whether v is finite, nonzero and not subnormal as a float32."""
+    return 2.0 ** -126 <= abs(_f32(v)) < math.inf
+
+
 def _is_factor(e):
-    """A finite nonzero constant."""
-    return e.op == "const" and e.dtype != "b" and e.value != 0 and math.isfinite(float(e.value))
+    """A constant that is a normal float32."""
+    return e.op == "const" and e.dtype != "b" and _is_normal(e.value)
 
 
 def _mul(a, b):
-    # constant factors collect into one: the derivative of c tanh(s / c) is 1 - tanh^2
+    # constant factors collect into one where that is a normal float32: the
+    # derivative of c tanh(s / c) is 1 - tanh^2
     if _is_factor(a) and not _is_factor(b):
         a, b = b, a
     if _is_factor(b) and a.op == "mul" and a.dtype == "f":
         for x, k in (a.args, a.args[::-1]):
-            if _is_factor(k) and math.isfinite(float(k.value) * float(b.value)):
+            if _is_factor(k) and _is_normal(float(k.value) * float(b.value)):
                 return _mul(x, _fconst(float(k.value) * float(b.value)))
     if _is(a, 0.0) or _is(b, 0.0) or _is(a, 0) or _is(b, 0):
         return ZERO
@@ -451,8 +463,9 @@ def derivative(e: Expr) -> Expr:
     if op == "truediv":
         da, db = derivative(a[0]), derivative(a[1])
         if _is(db, 0.0) or _is(db, 0):  # a divisor without the score: (u / c)' = u' (1 / c)
-            inv = _fconst(1.0 / float(np.float32(a[1].value))) if _is_factor(a[1]) else binop("truediv", ONE, a[1])
-            return _mul(da, inv)
+            if _is_factor(a[1]) and _is_normal(1.0 / _f32(a[1].value)):
+                return _mul(da, _fconst(1.0 / _f32(a[1].value)))
+            return _mul(da, binop("truediv", ONE, a[1]))
         num = _add(_mul(da, a[1]), _mul(_fconst(-1), _mul(a[0], db)))
         return binop("truediv", num, binop("mul", a[1], a[1])) if not _is(num, 0.0) else ZERO
     if op == "neg":
@@ -541,7 +554,7 @@ def _reciprocal(e: Expr):
     its sign: an infinite dividend stays infinite in x hi + x lo."""
     if e.op != "const" or e.dtype == "b":
         return None
-    c = float(np.float32(e.value))
+    c = _f32(e.value)
     if not 2.0 ** -90 < abs(c) < 2.0 ** 90:
         return None
     hi = np.float32(1.0 / c)

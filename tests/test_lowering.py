@@ -3,6 +3,8 @@ evaluates like the callable itself, Python's integer semantics survive,
 derivatives with respect to the score match finite differences, untraceable
 callables are refused with a reason, and the generated policy compiles for
 gfx950 through the C ABI (fa_mods_compile needs no GPU)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -197,3 +199,24 @@ def test_shared_functions_and_constant_factors_are_emitted_once():
     assert "*dsds = ((1.0f) - (t1 * t1));" in body
     # a divisor without a reciprocal in the normal range keeps its division
     assert "/ (0.0f)" in L.policy_source(None, L.lower_score(lambda s, b, h, q, kv: s / 0.0).expr)
+
+
+@pytest.mark.parametrize("name,fn", [
+    ("tiny_divisor", lambda s, b, h, q, kv: s / 1e-50),
+    ("huge_divisor", lambda s, b, h, q, kv: s / 1e300),
+    ("nested", lambda s, b, h, q, kv: torch.tanh(torch.tanh(s * 1e-30) * 1e-30) * 1e20 * 1e20 * 1e20),
+    ("growing", lambda s, b, h, q, kv: torch.tanh(torch.tanh(s * 1e30) * 1e30) * 1e-20),
+    ("subnormal", lambda s, b, h, q, kv: torch.sin(torch.sin(s * 1e-20) * 1e-20) + s),
+    ("divisors", lambda s, b, h, q, kv: torch.tanh(s / 1e30) / 1e-30 / 1e-30)])
+def test_folded_constants_stay_in_float32(name, fn):
+    """Constant factors of a derivative are folded only where their product is a normal float32: the emitted
+    code holds no literal that the program did not write and that is 0, subnormal or infinite in float32."""
+    expr = L.lower_score(fn).expr
+    src = L.policy_source(None, expr)
+    body = src[src.index("struct UserMod"):]
+    written = {float(x) for x in re.findall(r"(?<![\w.])(\d+\.?\d*(?:e[-+]?\d+)?)f", L.emit(expr))}
+    for text in re.findall(r"(?<![\w.])(\d+\.?\d*(?:e[-+]?\d+)?)f", body):
+        v = float(text)
+        with np.errstate(over="ignore", under="ignore"):
+            f = np.float32(v)
+        assert v == 0 or v in written or (np.isfinite(f) and abs(f) >= np.finfo(np.float32).tiny), (text, body)
