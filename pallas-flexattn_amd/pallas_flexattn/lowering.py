@@ -437,10 +437,12 @@ def _mul(a, b):
                 return _mul(x, _fconst(float(k.value) * float(b.value)))
     if _is(a, 0.0) or _is(b, 0.0) or _is(a, 0) or _is(b, 0):
         return ZERO
+    # (1.0 times an integer is a float: a product of two positions left as
+    # integers can pass 2^31)
     if _is(a, 1.0):
-        return b
+        return b if b.dtype == "f" else unop("float", b)
     if _is(b, 1.0):
-        return a
+        return a if a.dtype == "f" else unop("float", a)
     return binop("mul", a, b)
 
 

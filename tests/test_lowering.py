@@ -220,3 +220,12 @@ def test_folded_constants_stay_in_float32(name, fn):
         with np.errstate(over="ignore", under="ignore"):
             f = np.float32(v)
         assert v == 0 or v in written or (np.isfinite(f) and abs(f) >= np.finfo(np.float32).tiny), (text, body)
+
+
+def test_derivative_of_integer_factors_is_a_float_product():
+    for fn in (lambda s, b, h, q, kv: s * (kv * 0.5) * 2.0 * q, lambda s, b, h, q, kv: s * kv * q):
+        low = L.lower_score(fn)
+        n = np.array([[70000]], dtype=np.int32)
+        np.testing.assert_allclose(low.grad(np.ones((1, 1), np.float32), 0, 0, n, n), 70000.0 ** 2, rtol=1e-6)
+        body = L.policy_source(None, low.expr)
+        assert "*dsds = (((float)(kv)) * ((float)(q)));" in body, body
