@@ -551,78 +551,88 @@ void fwd_bf16_kernel(FwdArgs a) {
 
 // Split-KV merge.  With the splits' partials O_s (relative to 2^m_s) and sums
 // l_s: M = max m_s, L = sum l_s 2^(m_s - M), O = sum O_s 2^(m_s - M) / L,
-// LSE = (M + log2 L) ln 2.  One wave per row takes up to 16 splits (lane s
-// holds split s's factor, the columns go over the lanes, loads eight splits
-// deep); with more, the four waves of a workgroup share one row's splits and
-// add up through LDS.  Bound by latency: a thread per element that walked the
-// splits one load at a time took 6.8 us for 256 rows of 8 splits and 20 us for
-// 32 rows of 64, this 3.1 and 4.5.
+// LSE = (M + log2 L) ln 2.  One wave per row takes up to 16 splits (lane s of
+// each 16 holds split s's factor, the columns go over the lanes, loads eight
+// splits deep, the first eight ahead of the factors); with more (kShared), the
+// four waves of a workgroup share one row's splits and add up through LDS.
+// Bound by latency: a thread per element that walked the splits one load at a
+// time took 6.8 us for 256 rows of 8 splits and 20 us for 32 rows of 64, this
+// 3.1 and 4.5.
 template <int D, bool kShared>
 __global__ __launch_bounds__(256) void fwd_split_merge(FwdArgs a) {
   constexpr int CPL = D >= 64 ? D / 64 : 1;  // columns per lane
+  constexpr int LS = kShared ? 64 : 16;      // lanes that hold the splits' factors
   __shared__ float sums[kShared ? 4 * D : 1];
   const Problem& P = a.p;
   const size_t rows = (size_t)P.B * P.Hq * P.Sq;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const size_t row = kShared ? (size_t)blockIdx.x : (size_t)blockIdx.x * 4 + w;
-  if (row >= rows) return;  // (wave-uniform; with kShared the grid has one workgroup per row)
   const int n = a.n_splits;
-  const float* pml = a.part + (size_t)n * rows * D;
-  float2 ml = make_float2(-INFINITY, 0.f);
-  if (lane < n) ml = *reinterpret_cast<const float2*>(pml + ((size_t)lane * rows + row) * 2);
-  float mm = ml.x;
-#pragma unroll
-  for (int x = 32; x >= 1; x >>= 1) mm = fmaxf(mm, __shfl_xor(mm, x, 64));
-  const float c = ml.x == -INFINITY ? 0.f : fast_exp2(ml.x - mm);
-  float L = ml.y * c;
-#pragma unroll
-  for (int x = 32; x >= 1; x >>= 1) L += __shfl_xor(L, x, 64);
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
   const int col = lane * CPL < D ? lane * CPL : 0;  // (D = 32: lanes 32 .. 63 repeat column 0)
-  float acc[CPL];
-#pragma unroll
-  for (int k = 0; k < CPL; ++k) acc[k] = 0.f;
-  const float* po = a.part + row * D + col;
   constexpr int STEP = kShared ? 4 : 1, DEEP = 8;
-  for (int s0 = kShared ? w : 0; s0 < n; s0 += STEP * DEEP) {
+  const int first = kShared ? w : 0;
+  // (kShared: a workgroup per row, else a wave per row; rows past the grid's end follow)
+  const size_t step = kShared ? (size_t)gridDim.x : (size_t)gridDim.x * 4;
+  for (size_t row = kShared ? (size_t)blockIdx.x : (size_t)blockIdx.x * 4 + w; row < rows; row += step) {
+    const float* pml = a.part + (size_t)n * rows * D;
+    const float* po = a.part + row * D + col;
     float x[DEEP][CPL];
+    auto load = [&](int s0) {
 #pragma unroll
-    for (int u = 0; u < DEEP; ++u) {
-      const int s = imin(s0 + u * STEP, n - 1);
-      const float* p = po + (size_t)s * rows * D;
-      if constexpr (CPL == 2) {
-        const float2 v = *reinterpret_cast<const float2*>(p);
-        x[u][0] = v.x;
-        x[u][1] = v.y;
-      } else {
-        x[u][0] = p[0];
+      for (int u = 0; u < DEEP; ++u) {
+        const float* p = po + (size_t)imin(s0 + u * STEP, n - 1) * rows * D;
+        if constexpr (CPL == 2) {
+          const float2 v = *reinterpret_cast<const float2*>(p);
+          x[u][0] = v.x;
+          x[u][1] = v.y;
+        } else {
+          x[u][0] = p[0];
+        }
+      }
+    };
+    float2 ml = make_float2(-INFINITY, 0.f);
+    if ((lane & (LS - 1)) < n) ml = *reinterpret_cast<const float2*>(pml + ((size_t)(lane & (LS - 1)) * rows + row) * 2);
+    load(first);
+    float mm = ml.x;
+#pragma unroll
+    for (int d = LS / 2; d >= 1; d >>= 1) mm = fmaxf(mm, __shfl_xor(mm, d, 64));
+    const float c = ml.x == -INFINITY ? 0.f : fast_exp2(ml.x - mm);
+    float L = ml.y * c;
+#pragma unroll
+    for (int d = LS / 2; d >= 1; d >>= 1) L += __shfl_xor(L, d, 64);
+    const float inv = L > 0.f ? 1.0f / L : 0.f;
+    float acc[CPL];
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) acc[k] = 0.f;
+    for (int s0 = first; s0 < n; s0 += STEP * DEEP) {
+      if (s0 != first) load(s0);
+#pragma unroll
+      for (int u = 0; u < DEEP; ++u) {
+        const int s = s0 + u * STEP;
+        // a split without a live key left its partial O unwritten
+        const float cs = __shfl(c, s & (LS - 1), 64);
+        const bool live = s < n && !(cs == 0.f);  // (NaN is passed on)
+#pragma unroll
+        for (int k = 0; k < CPL; ++k) acc[k] = live ? fmaf(x[u][k], cs, acc[k]) : acc[k];
       }
     }
+    if constexpr (kShared) {
 #pragma unroll
-    for (int u = 0; u < DEEP; ++u) {
-      const int s = s0 + u * STEP;
-      // a split without a live key left its partial O unwritten
-      const float cs = __shfl(c, s & 63, 64);
-      const bool live = s < n && !(cs == 0.f);  // (NaN is passed on)
+      for (int k = 0; k < CPL; ++k)
+        if (lane * CPL < D) sums[w * D + col + k] = acc[k];
+      __syncthreads();
 #pragma unroll
-      for (int k = 0; k < CPL; ++k) acc[k] = live ? fmaf(x[u][k], cs, acc[k]) : acc[k];
+      for (int k = 0; k < CPL; ++k)
+        acc[k] = (sums[col + k] + sums[D + col + k]) + (sums[2 * D + col + k] + sums[3 * D + col + k]);
+      __syncthreads();  // (before the next row's sums)
+      if (w) continue;
     }
+    if (lane * CPL < D) {
+      uint16_t* o = static_cast<uint16_t*>(a.o) + row * D + col;
+      if constexpr (CPL == 2) *reinterpret_cast<uint32_t*>(o) = pack_bf16x2(acc[0] * inv, acc[1] * inv);
+      else *o = (uint16_t)(pack_bf16x2(acc[0] * inv, 0.f) & 0xffffu);
+    }
+    if (lane == 0) a.lse[row] = L > 0.f ? (mm + log2f(L)) * kLn2 : -INFINITY;
   }
-  if constexpr (kShared) {
-#pragma unroll
-    for (int k = 0; k < CPL; ++k)
-      if (lane * CPL < D) sums[w * D + col + k] = acc[k];
-    __syncthreads();
-    if (w) return;
-#pragma unroll
-    for (int k = 0; k < CPL; ++k) acc[k] = (sums[col + k] + sums[D + col + k]) + (sums[2 * D + col + k] + sums[3 * D + col + k]);
-  }
-  if (lane * CPL < D) {
-    uint16_t* o = static_cast<uint16_t*>(a.o) + row * D + col;
-    if constexpr (CPL == 2) *reinterpret_cast<uint32_t*>(o) = pack_bf16x2(acc[0] * inv, acc[1] * inv);
-    else *o = (uint16_t)(pack_bf16x2(acc[0] * inv, 0.f) & 0xffffu);
-  }
-  if (lane == 0) a.lse[row] = L > 0.f ? (mm + log2f(L)) * kLn2 : -INFINITY;
 }
 
 }  // namespace fa

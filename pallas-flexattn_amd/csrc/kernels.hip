@@ -53,11 +53,11 @@ int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
                            dim3(NW * 64), 0, s, a);
       }
       if (a.n_splits > 1) {
-        const unsigned rows = (unsigned)a.p.B * a.p.Hq * a.p.Sq;
-        if (a.n_splits > 16)
-          hipLaunchKernelGGL((fa::fwd_split_merge<D, true>), dim3(rows), dim3(256), 0, s, a);
+        const dim3 merge(merge_grid(a.p, a.n_splits));
+        if (a.n_splits > kMergeWave)
+          hipLaunchKernelGGL((fa::fwd_split_merge<D, true>), merge, dim3(256), 0, s, a);
         else
-          hipLaunchKernelGGL((fa::fwd_split_merge<D, false>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+          hipLaunchKernelGGL((fa::fwd_split_merge<D, false>), merge, dim3(256), 0, s, a);
       }
       return launch_status();
     }

@@ -272,6 +272,16 @@ inline int choose_split_keys(const fa_params* p, const Problem& pr, int n_splits
   return cdiv(cdiv(p->Skv, n_splits), 64) * 64;
 }
 
+// Workgroups (256 threads) of the merge: a wave per row up to kMergeWave
+// splits, else a workgroup per row; the kernel walks the rows past a launch of
+// 2^23 workgroups (HIP takes fewer than 2^32 threads a launch).
+constexpr int kMergeWave = 16;
+inline unsigned merge_grid(const Problem& pr, int n_splits) {
+  const size_t rows = (size_t)pr.B * pr.Hq * pr.Sq;
+  const size_t wgs = n_splits > kMergeWave ? rows : (rows + 3) / 4;
+  return (unsigned)(wgs < (1u << 23) ? wgs : (1u << 23));
+}
+
 inline size_t split_bytes(const fa_params* p, int n) {
   return n > 1 ? (size_t)n * p->B * p->Hq * p->Sq * (p->D + 2) * sizeof(float) : 0;
 }

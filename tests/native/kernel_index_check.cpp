@@ -570,7 +570,24 @@ static int check_paged(const Case& c) {
   return 1;
 }
 
+// The merge's launch: fewer than 2^32 threads whatever the rows, a row per wave
+// or workgroup where they fit
+static void check_merge_grid() {
+  g_where = "merge grid";
+  for (long long rows : {1ll, 4ll, 5ll, 1ll << 22, (1ll << 24) - 1, 1ll << 24, (1ll << 26) + 3, (1ll << 30) + 1})
+    for (int n : {2, kMergeWave, kMergeWave + 1, 64}) {
+      Problem P{};
+      P.B = 1;
+      P.Hq = 1;
+      P.Sq = (int)rows;
+      const long long g = merge_grid(P, n), per = n > kMergeWave ? 1 : 4;
+      if (g < 1 || g * 256 >= 1ll << 32) fail("merge launch too large");
+      if (rows <= 1 << 22 && g * per < rows) fail("merge launch too small");
+    }
+}
+
 int main(int argc, char** argv) {
+  check_merge_grid();
   if (argc < 2) {
     std::fprintf(stderr, "usage: %s cases.bin\n", argv[0]);
     return 2;
