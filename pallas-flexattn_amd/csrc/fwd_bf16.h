@@ -161,8 +161,9 @@ void fwd_bf16_kernel(FwdArgs a) {
   [[maybe_unused]] const int chunk = a.split_keys / BN;
   // a split past a short row's keys has nothing to read: (m, l) = (-inf, 0),
   // its partial O is never looked at
+  SplitRange sr{0, n_it};
   if constexpr (kCache) {
-    const SplitRange sr = split_range(n_it, split, a.n_splits, chunk);
+    sr = split_range(n_it, split, a.n_splits, chunk);
     if (a.n_splits > 1 && sr.it0 >= sr.it1) {
       if (qvalid && hh == 0) {
         const size_t all_rows = (size_t)P.B * P.Hq * P.Sq;
@@ -301,7 +302,6 @@ void fwd_bf16_kernel(FwdArgs a) {
   const int n_full = walk.count_full();
   int it0, it1;
   if constexpr (kCache) {
-    const SplitRange sr = split_range(n_it, split, a.n_splits, chunk);
     it0 = sr.it0;
     it1 = sr.it1;
   } else {  // equal shares, written out: the shared form costs the unsplit forward 0.7 % (SGPR layout)
@@ -337,9 +337,10 @@ void fwd_bf16_kernel(FwdArgs a) {
     // a partial tile that no row of this wave sees (two of the eight wave tiles
     // of a diagonal block) only issues its copies: forward at D = 128, causal
     // S8192 2018 -> 1986 us, S2048 160 -> 157, window 1024 648 -> 631; at D = 64
-    // the test costs what it saves (and in dQ its registers: 209 -> 236 us, spills)
+    // the test costs what it saves (and in dQ its registers: 209 -> 236 us, spills),
+    // and decode has no such tiles (32 x 1 heads of 512 keys: 10.1 us with the test, 9.7 without)
     bool run = kbase < skv;
-    if constexpr (D == 128 && NS > 1 && !Mod::kMask) {  // (NS = 1 has a barrier inside)
+    if constexpr (D == 128 && NS > 1 && !Mod::kMask && !kCache) {  // (NS = 1 has a barrier inside)
       if (masked) run = run && __any(qvalid && klo <= kbase + BN - 1 && khi >= kbase);
     }
     if (NS > 1 && !run && more) {

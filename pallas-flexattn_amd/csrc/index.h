@@ -252,7 +252,10 @@ FA_HD SplitRange split_range(int n_it, int split, int n_splits, int chunk) {
     const int it0 = imin(split * chunk, n_it);
     return SplitRange{it0, imin(it0 + chunk, n_it)};
   }
-  return SplitRange{(int)((long long)n_it * split / n_splits), (int)((long long)n_it * (split + 1) / n_splits)};
+  // floor(n_it s / n_splits) without a 64-bit division (a hundred scalar
+  // instructions in front of a decode workgroup's first load)
+  const int q = n_it / n_splits, r = n_it - q * n_splits;
+  return SplitRange{q * split + r * split / n_splits, q * (split + 1) + r * (split + 1) / n_splits};
 }
 
 // A tile of a walk whose table entry may still be in flight: fetch() issues

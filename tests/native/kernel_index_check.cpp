@@ -570,6 +570,24 @@ static int check_paged(const Case& c) {
   return 1;
 }
 
+// split_range against its 64-bit form, and splits that cover the walk
+static void check_split_range() {
+  g_where = "split ranges";
+  for (long long n_it : {0ll, 1ll, 5ll, 63ll, 64ll, 65ll, 1000ll, 32767ll, 67108863ll, 67108864ll})
+    for (int n : {1, 2, 3, 7, 16, 17, 63, 64})
+      for (int chunk : {0, 1, 3, (int)((n_it + n - 1) / n)}) {
+        if (chunk > 0 && (long long)chunk * n < n_it) continue;  // the host's runs cover the walk
+        long long prev = 0;
+        for (int i = 0; i < n; ++i) {
+          const SplitRange r = split_range((int)n_it, i, n, chunk);
+          if (chunk == 0 && (r.it0 != n_it * i / n || r.it1 != n_it * (i + 1) / n)) fail("equal shares");
+          if (r.it0 != prev || r.it1 < r.it0) fail("splits leave a gap");
+          prev = r.it1;
+        }
+        if (prev != n_it) fail("splits do not cover the walk");
+      }
+}
+
 // The merge's launch: fewer than 2^32 threads whatever the rows, a row per wave
 // or workgroup where they fit
 static void check_merge_grid() {
@@ -587,6 +605,7 @@ static void check_merge_grid() {
 }
 
 int main(int argc, char** argv) {
+  check_split_range();
   check_merge_grid();
   if (argc < 2) {
     std::fprintf(stderr, "usage: %s cases.bin\n", argv[0]);
