@@ -221,9 +221,14 @@ int fwd_launch(const fa_params* p, const fa_kv_cache* kv, const void* q, const v
   const bool lens = kv && kv->kv_lens;
   a.n_splits = split ? choose_splits(p, t, a.p, n_splits, device_cus(), lens) : 1;
   a.split_keys = fa::choose_split_keys(p, a.p, a.n_splits, lens);
+  const bool one_wave = fa::one_wave_fwd(a.p, a.pack, p->D, device_cus());
+  t.one_wave = one_wave && a.n_splits > 1;
   // rows of different lengths: an XCD that took whole batch rows (the L2 order)
   // would get more or less work than the others, so the heads go round the XCDs
-  if (lens && fa::one_wave_fwd(a.p, a.pack, p->D)) a.p.xcd_remap = 0;
+  // (128 heads of up to 7552 keys, five splits, L2 order / this: 78 / 62 us; 768
+  // of 1152 unsplit 65 / 60, 256 of 256 8.3 / 8.0).  Unsplit, with fewer items
+  // than units, it only costs (64 heads of 256 keys 9.6 / 10.0).
+  if (lens && one_wave && (a.n_splits > 1 || fwd_items(a.p, a.pack, t.bm) >= device_cus())) a.p.xcd_remap = 0;
   if (a.n_splits > 1) {
     if (!workspace || workspace_bytes < split_bytes(p, a.n_splits) || !aligned16({workspace}))
       return FA_ERR_WORKSPACE;

@@ -28,7 +28,7 @@ constexpr bool f32_grouped() {
 }
 
 template <typename T, int D, int BN, int NW, bool M, int NS = 2>
-int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
+int run_fwd(const FwdArgs& a, const Tiles& t, hipStream_t s) {
   const int grid = fwd_items(a.p, a.pack, 32 * NW);
   if constexpr (sizeof(T) == 2) {
     if (interval_masks(a.p)) {  // bf16: LDS-DMA + transposing-read kernel
@@ -39,7 +39,7 @@ int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
         // half the LDS per workgroup; measured 5.72 against 5.40 TB/s of KV
         // reads at B8 Hq32 Hkv8 Skv32768 (a plain streaming read reaches
         // ~5.8).  Unsplit, its grid of one-wave workgroups is too small.
-        if (one_wave_fwd(a.p, a.pack, D) && a.n_splits > 1)
+        if (t.one_wave)
           hipLaunchKernelGGL((fa::fwd_bf16_kernel<D, 32, 1, M, fa::BuiltinMod, true>),
                              dim3(fwd_items(a.p, a.pack, 32) * a.n_splits), dim3(64), 0, s, a);
         else if (cache)
@@ -68,7 +68,7 @@ int run_fwd(const FwdArgs& a, hipStream_t s, [[maybe_unused]] int groups = 1) {
   if constexpr (sizeof(T) == 4) {
     const dim3 items(fwd_items(a.p, 0, 32 * NW));
     if constexpr (f32_grouped<D, NW>())
-      if (groups == 2) {
+      if (t.ng == 2) {
         hipLaunchKernelGGL((fa::fwd_f32_kernel<D, NW, M, fa::BuiltinMod, 2>), items, dim3(2 * NW * 64), 0, s, g);
         return launch_status();
       }
@@ -86,13 +86,13 @@ int launch_fwd(const FwdArgs& a, const Tiles& t, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     if constexpr (D >= 64) {
       // LDS stages: 3 with 32-key tiles, 1 with 128-key tiles, else 2
-      if (t.bn == 32) return t.ns == 3 ? run_fwd<T, D, 32, 4, M, 3>(a, s) : run_fwd<T, D, 32, 4, M>(a, s);
-      if (t.bn == 128) return t.ns == 1 ? run_fwd<T, D, 128, 4, M, 1>(a, s) : run_fwd<T, D, 128, 4, M>(a, s);
-      if (t.bm == 256) return run_fwd<T, D, 64, 8, M>(a, s);
+      if (t.bn == 32) return t.ns == 3 ? run_fwd<T, D, 32, 4, M, 3>(a, t, s) : run_fwd<T, D, 32, 4, M>(a, t, s);
+      if (t.bn == 128) return t.ns == 1 ? run_fwd<T, D, 128, 4, M, 1>(a, t, s) : run_fwd<T, D, 128, 4, M>(a, t, s);
+      if (t.bm == 256) return run_fwd<T, D, 64, 8, M>(a, t, s);
     }
-    return t.bm == 64 ? run_fwd<T, D, 64, 2, M>(a, s) : run_fwd<T, D, 64, 4, M>(a, s);
+    return t.bm == 64 ? run_fwd<T, D, 64, 2, M>(a, t, s) : run_fwd<T, D, 64, 4, M>(a, t, s);
   } else {
-    return t.bm == 64 ? run_fwd<T, D, 32, 2, M>(a, s) : run_fwd<T, D, 32, 4, M>(a, s, t.ng);
+    return t.bm == 64 ? run_fwd<T, D, 32, 2, M>(a, t, s) : run_fwd<T, D, 32, 4, M>(a, t, s);
   }
 }
 

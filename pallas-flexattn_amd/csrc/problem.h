@@ -19,6 +19,7 @@ struct Tiles {
   int bkv, bq;   // dK/dV: key tile, query tile
   int ns;        // forward: K / V tiles held in LDS (stages)
   int ng = 1;    // float32 forward / dQ: groups of waves that share a work item (f32_groups)
+  bool one_wave = false;  // bf16 split forward: one-wave workgroups (one_wave_fwd)
 };
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -235,29 +236,47 @@ inline int choose_pack(const fa_params* p, const Tiles& t, const Problem& pr) {
 }
 
 // Decode shapes: every row of a work item in one 32-row block (g * Sq packed
-// rows, or Sq), which the split forward runs as one wave per workgroup.
-inline bool one_wave_fwd(const Problem& pr, int pack, int D) {
-  return D >= 64 && (pack > 1 ? pack : 1) * pr.Sq <= 32;
+// rows, or Sq), which the split forward can run as one wave per workgroup.
+// Ungrouped heads do so only where their 256-key runs (the shortest splits)
+// are more than the compute units (cus): with at most one workgroup per unit a
+// call is as long as one run's chain of tiles, and four waves on 64-key tiles
+// halve that chain.  Four waves / one wave (us, D128, equal lengths): 32 heads
+// of 512 keys 11.5 / 12.6, 128 of 512 13.7 / 14.9, 8 of 1152 11.5 / 12.6 (D64,
+// 32 of 512: 9.7 / 10.4); above the line 32 of 2432 16.4 / 16.3, 384 of 640
+// 33.2 / 30.5, 384 of 2432 92 / 87 (D64, 128 of 1152: 14.0 / 13.2).
+inline bool one_wave_fwd(const Problem& pr, int pack, int D, int cus) {
+  if (D < 64 || (pack > 1 ? pack : 1) * pr.Sq > 32) return false;
+  return pack > 1 || (long long)fwd_items(pr, 0, 128) * cdiv(pr.Skv, 256) > cus;
 }
 
 // Split-KV: the requested count, or 1 where the generic kernel runs.  <= 0:
 // as many as give a CU (of cus) two workgroups, at least four key tiles per
-// split.  The one-wave workgroups of decode shapes take more: a tile in flight
-// is half as many bytes at D = 64 (four: B16 Hq32 Hkv4 Skv8192 27 us against
-// 40 with one, 27 with two to eight; B6 H4 Skv16640 21 against 25 with two),
-// and rows of different lengths (`lens`) balance over five (B32 Hq32 Hkv8
-// Skv8192 D128, lengths of a tenth and more: 144 / 115 / 104 / 122 us with 2 /
-// 3 / 5 / 8; B18 Hq128 Hkv16 Skv10368 D64 160 / 118 / 91 / 100).  With equal
-// lengths at D = 128 more than two only cost merging (B8 Hq32 Hkv8 Skv32768:
-// 184 / 191 / 205 us with 2 / 3 / 6).
+// split.  The one-wave workgroups of decode shapes:
+// * equal lengths, D = 64, three: a tile in flight is half as many bytes
+//   (128 heads of 30464 keys, 500 MB, with 1 / 2 / 3 / 4: 191 / 111 / 87 / 90 us);
+//   at D = 128 more than two only cost merging (B8 Hq32 Hkv8 Skv32768:
+//   184 / 191 / 205 us with 2 / 3 / 6);
+// * rows of different lengths (`lens`) balance over five (32 x 8 kv heads of up
+//   to 8192 keys at D = 128: 144 / 115 / 104 / 122 us with 2 / 3 / 5 / 8), four
+//   below one item per CU at D = 128 (32 heads of up to 30464 keys with 3 / 4 / 5:
+//   73 / 73 / 89 us, 64 of 15232: 74 / 74 / 88, 128 of 7552: 62 / 63 / 62);
+// * from two items per CU on, two splits are none: 512 items with 1 / 2 43 / 47
+//   us (D64, 1792 keys), lengths at D = 128 (896 keys) 31.5 / 35.1, 768 items with
+//   lengths at D = 64 (1152 keys) 31.3 / 33.8, but up to 1024 keys 20.8 / 19.4 (640);
+//   three only at D = 64 with lengths (512 items: 13 % faster than one).
 inline int choose_splits(const fa_params* p, const Tiles& t, const Problem& pr, int requested, int cus, bool lens) {
   if (p->dtype != FA_DTYPE_BF16 || !interval_masks(pr)) return 1;
   const int pack = choose_pack(p, t, pr);
   const int items = fwd_items(pr, pack, t.bm);
   const int max_by_keys = cdiv(p->Skv, 4 * t.bn);
-  const int per_cu = !one_wave_fwd(pr, pack, p->D) ? 2 : lens ? 5 : p->D < 128 ? 4 : 2;
+  int per_cu = 2;
+  if (one_wave_fwd(pr, pack, p->D, cus)) {
+    if (p->D < 128) per_cu = lens ? 5 : 3;
+    else if (lens && items < 2 * cus) per_cu = items < cus ? 4 : 5;
+  }
   int n = requested;
   if (n <= 0) n = cdiv(per_cu * cus, items);
+  if (requested <= 0 && n <= 2 && items >= 2 * cus && !(lens && p->D < 128 && p->Skv <= 1024)) n = 1;
   if (n > max_by_keys) n = max_by_keys;
   if (n > 64) n = 64;
   return n < 1 ? 1 : n;

@@ -448,7 +448,7 @@ static void model_dkdv(const Problem& P, int parts) {
 template <int D>
 static void run_fwd(const Problem& P, const Tiles& t, const FwdOpts& o) {
   if constexpr (D >= 64) {
-    if (o.n_splits > 1 && one_wave_fwd(P, o.pack, D) && t.bn == 64 && t.bm == 128) return model_fwd<D, 32, 1, 2>(P, o);
+    if (o.n_splits > 1 && one_wave_fwd(P, o.pack, D, 256) && t.bn == 64 && t.bm == 128) return model_fwd<D, 32, 1, 2>(P, o);
     if (t.bn == 32) return t.ns == 3 ? model_fwd<D, 32, 4, 3>(P, o) : model_fwd<D, 32, 4, 2>(P, o);
     if (t.bn == 128) return t.ns == 1 ? model_fwd<D, 128, 4, 1>(P, o) : model_fwd<D, 128, 4, 2>(P, o);
     if (t.bm == 256) return model_fwd<D, 64, 8, 2>(P, o);
@@ -604,9 +604,48 @@ static void check_merge_grid() {
     }
 }
 
+// Splits and workgroup form of decode calls on 256 compute units
+static void check_decode_rule() {
+  g_where = "decode rule";
+  struct Row {
+    int B, Hq, Hkv, Sq, Skv, D, lens, splits, one_wave;
+  };
+  const Row rows[] = {
+      {4, 8, 8, 1, 512, 128, 0, 2, 0},     {16, 8, 8, 1, 512, 128, 0, 2, 0},    {16, 8, 8, 1, 513, 128, 0, 3, 1},
+      {16, 8, 8, 1, 512, 64, 1, 2, 0},     {4, 8, 8, 32, 2432, 128, 1, 10, 1},  {4, 8, 8, 33, 2432, 128, 1, 10, 0},
+      {4, 32, 4, 1, 512, 128, 0, 2, 1},    {8, 32, 8, 1, 32768, 128, 0, 8, 1},  {32, 32, 8, 1, 8192, 128, 1, 5, 1},
+      {16, 32, 4, 1, 15232, 128, 1, 16, 1}, {16, 32, 4, 1, 30464, 64, 1, 20, 1}, {16, 32, 4, 1, 30464, 64, 0, 12, 1},
+      {32, 64, 16, 1, 1792, 64, 0, 1, 1},  {32, 64, 16, 1, 1792, 64, 1, 3, 1},  {32, 64, 16, 1, 896, 128, 1, 1, 1},
+      {48, 64, 16, 1, 1024, 64, 1, 2, 1},  {48, 64, 16, 1, 1025, 64, 1, 1, 1},  {1, 2, 2, 1, 65536, 32, 1, 64, 0},
+      {64, 128, 128, 1, 4096, 128, 0, 1, 1}};
+  for (const Row& r : rows) {
+    fa_params p{};
+    p.abi_version = FA_ABI_VERSION;
+    p.dtype = FA_DTYPE_BF16;
+    p.B = r.B;
+    p.Hq = r.Hq;
+    p.Hkv = r.Hkv;
+    p.Sq = r.Sq;
+    p.Skv = r.Skv;
+    p.D = r.D;
+    p.window_left = p.window_right = -1;
+    Tiles t;
+    Problem P;
+    if (default_tiles(&p, &t) != FA_OK || build_problem(&p, t, &P) != FA_OK) fail("problem");
+    const int n = choose_splits(&p, t, P, 0, 256, r.lens != 0);
+    const bool w = one_wave_fwd(P, choose_pack(&p, t, P), r.D, 256);
+    if (n != r.splits || w != (r.one_wave != 0)) {
+      std::fprintf(stderr, "B%d Hq%d Hkv%d Sq%d Skv%d D%d lens %d: %d splits, one wave %d\n", r.B, r.Hq, r.Hkv, r.Sq, r.Skv,
+                   r.D, r.lens, n, (int)w);
+      fail("decode rule");
+    }
+  }
+}
+
 int main(int argc, char** argv) {
   check_split_range();
   check_merge_grid();
+  check_decode_rule();
   if (argc < 2) {
     std::fprintf(stderr, "usage: %s cases.bin\n", argv[0]);
     return 2;

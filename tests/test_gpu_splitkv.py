@@ -232,3 +232,23 @@ def test_rows_of_different_lengths(Hq, Hkv, Sq, D, lens, splits):
         wo, wl = _oracle(q[b:b + 1], k[b:b + 1, :, :n], v[b:b + 1, :, :n])
         np.testing.assert_allclose(o[b:b + 1], wo, atol=2e-2, rtol=2e-2)
         np.testing.assert_allclose(lse[b:b + 1], wl, atol=1e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("Skv", [512, 513])
+@pytest.mark.parametrize("lens", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,Sq,D", [(8, 8, 1, 128), (8, 8, 32, 64), (32, 4, 1, 128)])
+def test_decode_workgroup_forms(Hq, Hkv, Sq, D, lens, Skv):
+    """Either side of the rule that gives ungrouped heads one-wave workgroups (more 256-key runs than
+    compute units: 16 x 8 heads of 513 keys), with and without lengths, against the oracle."""
+    import torch
+    import pallas_flexattn as pf
+    B = 16
+    q, k, v = _case(B, Hq, Hkv, Sq, Skv, D, 23)
+    n = [Skv, 1, 255, 257, 64, 300, 512, 31] * 2 if lens else None
+    o, lse = pf.flex_decode(q, k, v, enable_gqa=Hq != Hkv, return_lse=True,
+                            kv_lens=torch.tensor(n, dtype=torch.int32) if lens else None)
+    for b in (0, 1, 2, 3, 13, 15):
+        m = n[b] if lens else Skv
+        wo, wl = _oracle(q[b:b + 1], k[b:b + 1, :, :m], v[b:b + 1, :, :m])
+        np.testing.assert_allclose(o[b:b + 1].float().cpu().numpy(), wo, atol=2e-2, rtol=2e-2)
+        np.testing.assert_allclose(lse[b:b + 1].cpu().numpy(), wl, atol=1e-3, rtol=1e-3)
