@@ -41,7 +41,12 @@ struct BlobHeader {
 
 // Kernel instantiations for a policy: the bf16 tile kernels (128-query
 // forward / dQ tiles of 64 keys, 128-key dK/dV tiles of 64 queries) or the
-// float32 split kernels (32-row tiles).
+// float32 split kernels (32-row tiles).  dK/dV in float32 at D = 128 runs the
+// general kernel: the split one fills all 512 registers by itself, and with a
+// policy's registers spilled on top the compiler (LLVM 22) crashed on two of
+// eight policies tried, in the pass that rewrites MFMA copies after spilling.
+// (Built-in masks: 680 us with the general kernel, 428 with the split one at
+// B2 H16 S2048 causal.)
 std::vector<std::string> mod_kernels(int dtype, int D, bool mods) {
   const std::string d = std::to_string(D), m = mods ? "true" : "false";
   if (dtype == FA_DTYPE_BF16)
@@ -49,7 +54,8 @@ std::vector<std::string> mod_kernels(int dtype, int D, bool mods) {
             "fa::dq_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>",
             "fa::dkdv_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>"};
   return {"fa::fwd_f32_kernel<" + d + ", 4, " + m + ", UserMod>", "fa::dq_f32_kernel<" + d + ", 4, " + m + ", UserMod>",
-          "fa::dkdv_f32_kernel<" + d + ", 4, " + m + ", UserMod>"};
+          D == 128 ? "fa::dkdv_kernel<float, 128, 32, 4, " + m + ", UserMod>"
+                   : "fa::dkdv_f32_kernel<" + d + ", 4, " + m + ", UserMod>"};
 }
 
 void copy_log(const std::string& text, char* log, size_t log_bytes) {

@@ -77,6 +77,7 @@ CASES = [
     ("quadratic-score-window", "bf16", 1, 2, 2, 256, 32),
     ("softsign-causal", "bf16", 1, 4, 2, 320, 64),
     ("softsign-causal", "fp32", 1, 2, 2, 200, 64),
+    ("head-bias-table", "fp32", 1, 4, 2, 200, 128),
 ]
 
 

@@ -229,3 +229,20 @@ def test_derivative_of_integer_factors_is_a_float_product():
         np.testing.assert_allclose(low.grad(np.ones((1, 1), np.float32), 0, 0, n, n), 70000.0 ** 2, rtol=1e-6)
         body = L.policy_source(None, low.expr)
         assert "*dsds = (((float)(kv)) * ((float)(q)));" in body, body
+
+
+@pytest.mark.parametrize("name", ["tables", "functions"])
+def test_float32_policies_with_many_registers_compile(name):
+    """float32 at D = 128, where the kernels leave a policy the fewest registers: two table reads with a tanh, and
+    a sum of several functions (the compiler crashed on both next to a dK/dV kernel that fills the register file)."""
+    from pallas_flexattn import _lib
+    t = torch.rand(2, 4, 64, 64)
+    mask, score = {
+        "tables": (lambda b, h, q, kv: t[b, h, q % 64, kv % 64] > 0.3,
+                   lambda s, b, h, q, kv: s * t[b, h, kv % 64, q % 64] + t[b, h, q % 64, kv % 64] + 10 * torch.tanh(s / 10)),
+        "functions": (lambda q, kv: ((q // 3) % 5 != (kv // 7) % 5) | (q == kv),
+                      lambda s, b, h, q, kv: torch.log(torch.sigmoid(s) + 1.0)
+                      + torch.sqrt(s * s + 1.0) * torch.exp(-torch.abs(q - kv) / 64.0) + torch.sin(s)),
+    }[name]
+    mods = L.UserMods(L.lower_mask(mask), L.lower_score(score))
+    assert len(_lib.compile_mods(mods.source, _lib.DTYPE_F32, 128, mods.flags(False))) > 1000
