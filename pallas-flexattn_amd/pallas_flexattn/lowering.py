@@ -677,18 +677,23 @@ __device__ __forceinline__ float um_sq(float x) { return x * x; }
 __device__ __forceinline__ float um_mul2(float x, float hi, float lo) { return fmaf(x, hi, x * lo); }
 // tanh without branches.  The math library's tanhf is a divergent branch over
 // two long paths, evaluated per score: the forward and backward of a tanh cap
-// through it took 819 us at B4 H16 S2048 D64 (prefix mask), 422 with this
-// one (366 with the built-in soft-cap).  |x| >= 0.5: 1 - 2 / (2^(2 |x| log2 e) + 1) on the
-// exponential and reciprocal units; below, where that cancels, an odd
-// polynomial (minimax in x^2, 2^-26 relative).  Within 4 * 2^-24 relative.
+// through it took 819 us at B4 H16 S2048 D64 (prefix mask), 423 with this
+// one (366 with the built-in soft-cap).  |x| >= 0.8: 1 - 2 / (2^(2 |x| log2 e) + 1)
+// on the exponential and reciprocal units; below, where that cancels, an odd
+// polynomial (minimax in x^2, its first coefficient the float nearest -1/3).
+// Errors in units of 2^-24 of the value, this / the library's: largest 2.4 / 2.5,
+// root mean square up to 0.3 0.43 / 0.43, up to 1 0.49 / 0.52, up to 3 0.40 / 0.40
+// (the line at 0.5 and two terms less: largest 3.8, 0.46, 0.64, 0.46).
 __device__ __forceinline__ float um_tanh(float x) {
   const float a = fabsf(x), y = x * x;
   const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a * 2.8853900817779268f) + 1.0f);
   const float big = fmaf(-2.0f, r, 1.0f);
-  float p = fmaf(0.01725698875064151f, y, -0.05305294934872954f);
-  p = fmaf(p, y, 0.13325987273043643f);
-  p = fmaf(p, y, -0.33333148377139477f);
-  return a < 0.5f ? fmaf(x * y, p, x) : copysignf(big, x);
+  float p = fmaf(0.0016673924401402473f, y, -0.007573986891657114f);
+  p = fmaf(p, y, 0.02142648957669735f);
+  p = fmaf(p, y, -0.053895365446805954f);
+  p = fmaf(p, y, 0.13332898914813995f);
+  p = fmaf(p, y, -0.3333333432674408f);
+  return a < 0.8f ? fmaf(x * y, p, x) : copysignf(big, x);
 }
 __device__ __forceinline__ float um_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 }  // namespace um
