@@ -25,13 +25,24 @@
 // workgroup that stages it), P and dS in registers.  Everything else (softmax,
 // sums, Delta, the accumulators) is float32 as before.
 //
-// Range: partial products of infinities and NaN differ from the float32
-// product (inf times an exact zero piece), and huge values could overflow in a
-// piece, so a work item that meets an input of magnitude >= 2^30 discards what
-// it has and runs again on the float32 matrix instructions (fwd_item, dq_item,
-// dkdv_item: the general kernels' code, same results as a call without the
-// split).  Pieces below 2^-126 vanish: an absolute error at float32's own
-// underflow threshold.
+// Small values: bf16 has float32's exponents, so the low pieces of a value
+// below 2^-110 would fall off the end of them (2^-133).  Operands are therefore
+// scaled by 2^16 as they are split, which makes the pieces of every float32
+// exact, subnormal ones too, and the sums are scaled back (exactly) by 2^-32
+// where they are used: in the exponent's FMA, in dP - Delta, at the end.  Only
+// the forward's Q and K stay as they are: what their scores lose is below 2^-84
+// before the exponential.  Same results bit for bit at ordinary magnitudes;
+// unscaled / scaled, one board (us; forward, dK/dV, dQ): 45.5, 94, 59 / 47, 95, 61
+// at the first shape above, 711, 1497, 982 / 733, 1506, 987 at the second.
+//
+// Large values: partial products of infinities differ from the float32 product
+// (inf times an exact zero piece), and sums of 2^32 times their value overflow
+// before float32 ones do.  A work item that meets an element of Q or K of
+// magnitude >= 2^43 (below that the scores stay finite), or whose O, dQ, dK or
+// dV sums are not finite at the end (which V, dO and everything after the
+// exponential shows up in), discards what it has and runs again on the float32
+// matrix instructions (fwd_item, dq_item, dkdv_item: the general kernels' code,
+// same results as a call without the split).
 //
 // One structure for all three kernels: NW waves, 32 rows (or keys) per wave
 // with their split operands in registers, tiles of 32 rows of the two streamed
@@ -52,7 +63,9 @@ struct Frag3 {  // eight consecutive k of a matrix operand, as three bf16 pieces
   u32x4 p[3];
 };
 
-constexpr float kSplitMax = 1073741824.0f;  // 2^30
+constexpr float kSplitMax = 8796093022208.0f;  // 2^43
+constexpr float kUp = 65536.0f;                // 2^16: the scale of every split operand
+constexpr float kDown = 1.0f / kUp, kDown2 = kDown * kDown;
 
 // Word j (elements 2 j, 2 j + 1) of the three pieces.  The packed words are
 // opaque to the compiler, which would otherwise convert each low element a
@@ -212,8 +225,9 @@ struct SplitStage {
       v[u][1] = buf_load16(rs, off + 16);
     }
   }
-  // half h (four floats) of chunk u split into its three planes; returns the
-  // largest magnitude seen
+  // half h (four floats) of chunk u split into its three planes; kMag: returns
+  // the largest magnitude seen (else mag)
+  template <bool kScaled, bool kMag>
   __device__ __forceinline__ float store(char* tile, int u, int h, int tid, float mag) const {
     const int g = tid + u * NW * 64;
     // (keeps the compiler from splitting the chunk, and so waiting for its
@@ -227,59 +241,83 @@ struct SplitStage {
       x[t] = __uint_as_float(word);
     }
     Frag3 f;
-    split2(f, 0, x[0], x[1]);
-    split2(f, 1, x[2], x[3]);
+    const float up = kScaled ? kUp : 1.0f;
+    split2(f, 0, x[0] * up, x[1] * up);
+    split2(f, 1, x[2] * up, x[3] * up);
     if (Tile::kAll || g < Tile::kChunks) {
       const int row = g / Tile::KCH, c = g % Tile::KCH;
       char* p = tile + row * Tile::RB + ((c ^ chunk_swz<Tile::KCH>(row)) * 16) + 8 * h;
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2*>(p + i * Tile::kPlane) = u32x2{f.p[i][0], f.p[i][1]};
     }
-    return max_mag(max_mag(mag, x[0], x[1]), x[2], x[3]);
+    return kMag ? max_mag(max_mag(mag, x[0], x[1]), x[2], x[3]) : mag;
   }
 };
 
 // The halves of both streamed tensors that a tile's k step s splits (all of
-// them over the KS steps).
-template <int D, int NW>
+// them over the KS steps); x is the score's factor, whose magnitudes count, and
+// is scaled with kScaledX.
+template <int D, int NW, bool kScaledX = true>
 __device__ __forceinline__ float stage_step(const SplitStage<D, NW>& x, const SplitStage<D, NW>& y, char* xt, char* yt,
                                             int s, int tid, float mag) {
   constexpr int PER = SplitTile<D, NW>::kPer, N = 4 * PER, KS = D / 16;
   static_assert(N % KS == 0 || KS % N == 0, "halves over steps");
 #pragma unroll
   for (int u = s * N / KS; u < (s + 1) * N / KS; ++u) {
-    if (u < 2 * PER) mag = x.store(xt, u >> 1, u & 1, tid, mag);
-    else mag = y.store(yt, (u - 2 * PER) >> 1, u & 1, tid, mag);
+    if (u < 2 * PER) mag = x.template store<kScaledX, true>(xt, u >> 1, u & 1, tid, mag);
+    else mag = y.template store<true, false>(yt, (u - 2 * PER) >> 1, u & 1, tid, mag);
   }
   return mag;
 }
 
-// A row operand kept in registers: row `row` of a (rows, D) tensor at base.
-template <int D>
+// A row operand kept in registers: row `row` of a (rows, D) tensor at base;
+// returns the largest magnitude seen.
+template <int D, bool kScaled = true>
 __device__ __forceinline__ float load_rows3(Frag3* f, const float* base, int row, bool ok, int hh, float mag) {
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) {
     const f32x8 v = ld_frag<float>(base + (size_t)row * D + 16 * s + 8 * hh, ok);
     float x[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) x[t] = v[t];
+    for (int t = 0; t < 8; ++t) x[t] = v[t] * (kScaled ? kUp : 1.0f);
     f[s] = split8(x);
 #pragma unroll
-    for (int t = 0; t < 8; t += 2) mag = max_mag(mag, x[t], x[t + 1]);
+    for (int t = 0; t < 8; t += 2) mag = max_mag(mag, v[t], v[t + 1]);
   }
   return mag;
 }
 
-// Whether any lane of the workgroup met an input that the split does not
-// take; `flag` is a word of LDS.  Ends with a barrier.
-__device__ __forceinline__ bool any_large(float mag, uint32_t* flag) {
+// Whether any lane of the workgroup met a score factor that the split does not
+// take, or sums that are not finite (`probe`: their products with 0, added up);
+// `flag` is a word of LDS.  Ends with a barrier.
+__device__ __forceinline__ bool any_large(float mag, float probe, uint32_t* flag) {
   __syncthreads();
   if (threadIdx.x == 0) *flag = 0u;
   __syncthreads();
-  if (mag >= kSplitMax) *flag = 1u;
+  if (mag >= kSplitMax || !(probe == 0.f)) *flag = 1u;
   __syncthreads();
   return *flag != 0u;
 }
+
+// 0 where every accumulator is finite, else NaN.
+template <int N>
+__device__ __forceinline__ float finite_probe(const f32x16* acc, float z) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z = fmaf(acc[i][e], 0.f, z);
+  return z;
+}
+
+// A gradient's last factors (2^-32 and the softmax scale), the smaller first:
+// the product neither overflows before it is due nor rounds twice unless it is
+// subnormal.
+struct GradScale {
+  float a, b;
+  __device__ __forceinline__ explicit GradScale(float scale)
+      : a(scale > 1.0f ? kDown2 : scale), b(scale > 1.0f ? scale : kDown2) {}
+  __device__ __forceinline__ float operator()(float x) const { return x * a * b; }
+};
 
 // A group's accumulators in LDS, one column per thread: x = base + thread.
 template <int N, int NW>
@@ -351,7 +389,7 @@ __device__ __forceinline__ bool fwd_split_item(const FwdArgs& a, char* lds, uint
   };
   load_tile(kb_c);
   Frag3 qf[KS];
-  float mag = load_rows3<D>(qf, static_cast<const float*>(a.q) + (size_t)head * P.Sq * D, qw, qvalid, hh, 0.f);
+  float mag = load_rows3<D, false>(qf, static_cast<const float*>(a.q) + (size_t)head * P.Sq * D, qw, qvalid, hh, 0.f);
   const float slope = P.alibi ? P.alibi[h] : 0.f;
   ElemMask em;
   em.interval = interval_mask(P);
@@ -366,7 +404,7 @@ __device__ __forceinline__ bool fwd_split_item(const FwdArgs& a, char* lds, uint
   float m = -INFINITY, l = 0.f;
 
   auto stage_kv = [&](int buf, int st) {
-    mag = stage_step<D, NW>(ks, vs, tiles + buf * TB, tiles + (2 + buf) * TB, st, tid, mag);
+    mag = stage_step<D, NW, false>(ks, vs, tiles + buf * TB, tiles + (2 + buf) * TB, st, tid, mag);
   };
 #pragma unroll
   for (int st = 0; st < KS; ++st) stage_kv(0, st);
@@ -446,7 +484,7 @@ __device__ __forceinline__ bool fwd_split_item(const FwdArgs& a, char* lds, uint
       const float y = fast_exp2(fmaf(sacc[8 * c + 2 * j + 1], sc, -muse));
       r0 += x;
       r1 += y;
-      split2(pf[c], j, x, y);
+      split2(pf[c], j, x * kUp, y * kUp);
     };
 #pragma unroll
     for (int j = 0; j < 4; ++j) exps(0, j);
@@ -474,7 +512,7 @@ __device__ __forceinline__ bool fwd_split_item(const FwdArgs& a, char* lds, uint
   }
   if (it < n_it) tile_step(it + grp, Int<0>{});
 
-  if (any_large(mag, flag)) return false;
+  if (any_large(mag, qvalid ? finite_probe<DT>(oacc, 0.f) : 0.f, flag)) return false;
   if constexpr (NG > 1) {  // group 1's (m, l, O) through LDS, merged by group 0
     float* x = reinterpret_cast<float*>(lds) + tid;
     if (grp) {
@@ -495,7 +533,7 @@ __device__ __forceinline__ bool fwd_split_item(const FwdArgs& a, char* lds, uint
       for (int e = 0; e < 16; ++e) oacc[i][e] = oacc[i][e] * c0 + x[(i * 16 + e) * NW * 64] * c1;
   }
   const float lt = pair_sum(l);
-  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  const float inv = lt > 0.f ? kDown2 / lt : 0.f;
   if (qvalid) {
     float* op = static_cast<float*>(a.o) + ((size_t)head * P.Sq + qw) * D;
 #pragma unroll
@@ -564,12 +602,12 @@ __device__ __forceinline__ bool dq_split_item(const BwdArgs& a, char* lds, uint3
   Frag3 qf[KS], df[KS];
   const size_t qoff = (size_t)head * P.Sq * D;
   float mag = load_rows3<D>(qf, static_cast<const float*>(a.q) + qoff, qw, qvalid, hh, 0.f);
-  mag = load_rows3<D>(df, static_cast<const float*>(a.dout) + qoff, qw, qvalid, hh, mag);
+  load_rows3<D>(df, static_cast<const float*>(a.dout) + qoff, qw, qvalid, hh, 0.f);
   const size_t rowi = (size_t)head * P.Sq + qw;
   // a row with no live key (LSE = -inf) gets P = 0 everywhere, like rows past Sq
   const float lse_row = qvalid ? a.lse[rowi] : -INFINITY;
   const float lse2 = lse_row > -INFINITY ? lse_row * kLog2e : INFINITY;
-  const float dl = qvalid ? a.delta[rowi] : 0.f;
+  const float dl = qvalid ? a.delta[rowi] * kUp : 0.f;
   const float slope = P.alibi ? P.alibi[h] : 0.f;
   ElemMask em;
   em.interval = interval_mask(P);
@@ -609,7 +647,7 @@ __device__ __forceinline__ bool dq_split_item(const BwdArgs& a, char* lds, uint3
     if constexpr (kMods) {
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        sacc[e] = mod_score_t<Mod, kMods>(P, sacc[e], slope, b, h, qw, kbase + acc_row(e, hh), &dsdx[e]);
+        sacc[e] = mod_score_t<Mod, kMods>(P, sacc[e] * kDown2, slope, b, h, qw, kbase + acc_row(e, hh), &dsdx[e]);
     }
     if (masked) {
       if (em.interval) {
@@ -642,14 +680,14 @@ __device__ __forceinline__ bool dq_split_item(const BwdArgs& a, char* lds, uint3
         }
       }
     }
-    const float sc = kMods ? 1.0f : P.scale_log2;
+    const float sc = kMods ? 1.0f : P.scale_log2 * kDown2;
     Frag3 sf[2];
-    auto grads = [&](int c, int j) {  // dS of elements 8 c + 2 j, + 1, split
+    auto grads = [&](int c, int j) {  // 2^16 dS of elements 8 c + 2 j, + 1, split
       float y[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int e = 8 * c + 2 * j + t;
-        y[t] = fast_exp2(fmaf(sacc[e], sc, -lse2)) * (pacc[e] - dl);
+        y[t] = fast_exp2(fmaf(sacc[e], sc, -lse2)) * fmaf(pacc[e], kDown, -dl);
         if constexpr (kMods) y[t] *= dsdx[e];
       }
       split2(sf[c], j, y[0], y[1]);
@@ -679,7 +717,7 @@ __device__ __forceinline__ bool dq_split_item(const BwdArgs& a, char* lds, uint3
   }
   if (it < n_it) tile_step(it + grp, Int<0>{});
 
-  if (any_large(mag, flag)) return false;
+  if (any_large(mag, qvalid ? finite_probe<DT>(dqa, 0.f) : 0.f, flag)) return false;
   if constexpr (NG > 1) {
     float* x = reinterpret_cast<float*>(lds) + tid;
     if (grp) put_acc<DT, NW>(x, dqa);
@@ -689,13 +727,13 @@ __device__ __forceinline__ bool dq_split_item(const BwdArgs& a, char* lds, uint3
   }
   if (qvalid) {
     float* dqp = static_cast<float*>(a.dq) + rowi * D;
+    const GradScale gs(P.scale);
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<f32x4*>(dqp + 32 * i + 8 * j + 4 * hh) =
-            f32x4{dqa[i][4 * j] * P.scale, dqa[i][4 * j + 1] * P.scale, dqa[i][4 * j + 2] * P.scale,
-                  dqa[i][4 * j + 3] * P.scale};
+            f32x4{gs(dqa[i][4 * j]), gs(dqa[i][4 * j + 1]), gs(dqa[i][4 * j + 2]), gs(dqa[i][4 * j + 3])};
   }
   return true;
 }
@@ -787,7 +825,7 @@ __device__ __forceinline__ bool dkdv_split_item(const BwdArgs& a, char* lds, flo
   fetch(grp + NG);
   Frag3 kf[KS], vf[KS];
   float mag = load_rows3<D>(kf, static_cast<const float*>(a.k) + (size_t)head * P.Skv * D, kw, kvalid, hh, 0.f);
-  mag = load_rows3<D>(vf, static_cast<const float*>(a.v) + (size_t)head * P.Skv * D, kw, kvalid, hh, mag);
+  load_rows3<D>(vf, static_cast<const float*>(a.v) + (size_t)head * P.Skv * D, kw, kvalid, hh, 0.f);
   ElemMask em;
   em.interval = interval_mask(P);
   query_interval(P, b, kw, &em.lo, &em.hi);
@@ -844,7 +882,7 @@ __device__ __forceinline__ bool dkdv_split_item(const BwdArgs& a, char* lds, flo
     if constexpr (kMods) {
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        sacc[e] = mod_score_t<Mod, kMods>(P, sacc[e], slope, b, hq, qbase + acc_row(e, hh), kw, &dsdx[e]);
+        sacc[e] = mod_score_t<Mod, kMods>(P, sacc[e] * kDown2, slope, b, hq, qbase + acc_row(e, hh), kw, &dsdx[e]);
     }
     if (masked) {
       if (em.interval) {
@@ -877,15 +915,15 @@ __device__ __forceinline__ bool dkdv_split_item(const BwdArgs& a, char* lds, flo
         }
       }
     }
-    const float sc = kMods ? 1.0f : P.scale_log2;
+    const float sc = kMods ? 1.0f : P.scale_log2 * kDown2;
     Frag3 pf[R], sf[R];
-    auto grads = [&](int c, int j) {  // P and dS (rows = queries, column = this lane's key), split
+    auto grads = [&](int c, int j) {  // 2^16 P and 2^16 dS (rows = queries, column = this lane's key), split
       float x[2], y[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int e = 8 * c + 2 * j + t;
-        x[t] = fast_exp2(fmaf(sacc[e], sc, -ls[e >> 2][e & 3]));
-        y[t] = x[t] * (pacc[e] - dd[e >> 2][e & 3]);
+        x[t] = fast_exp2(fmaf(sacc[e], sc, -ls[e >> 2][e & 3])) * kUp;
+        y[t] = x[t] * fmaf(pacc[e], kDown2, -dd[e >> 2][e & 3]);
         if constexpr (kMods) y[t] *= dsdx[e];
       }
       split2(pf[c % R], j, x[0], x[1]);
@@ -930,7 +968,7 @@ __device__ __forceinline__ bool dkdv_split_item(const BwdArgs& a, char* lds, flo
   }
   if (it < n_it) tile_step(it + grp, Int<0>{});
 
-  if (any_large(mag, flag)) return false;
+  if (any_large(mag, kvalid ? finite_probe<DT>(dva, finite_probe<DT>(dka, 0.f)) : 0.f, flag)) return false;
   if constexpr (NG > 1) {
     float* x = reinterpret_cast<float*>(lds) + tid;
     if (grp) {
@@ -945,15 +983,16 @@ __device__ __forceinline__ bool dkdv_split_item(const BwdArgs& a, char* lds, flo
   if (kvalid) {
     float* dkp = static_cast<float*>(a.dk) + ((size_t)head * P.Skv + kw) * D;
     float* dvp = static_cast<float*>(a.dv) + ((size_t)head * P.Skv + kw) * D;
+    const GradScale gs(P.scale), gv(1.0f);
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int d0 = 32 * i + 8 * j + 4 * hh;
-        *reinterpret_cast<f32x4*>(dkp + d0) = f32x4{dka[i][4 * j] * P.scale, dka[i][4 * j + 1] * P.scale,
-                                                    dka[i][4 * j + 2] * P.scale, dka[i][4 * j + 3] * P.scale};
+        *reinterpret_cast<f32x4*>(dkp + d0) =
+            f32x4{gs(dka[i][4 * j]), gs(dka[i][4 * j + 1]), gs(dka[i][4 * j + 2]), gs(dka[i][4 * j + 3])};
         *reinterpret_cast<f32x4*>(dvp + d0) =
-            f32x4{dva[i][4 * j], dva[i][4 * j + 1], dva[i][4 * j + 2], dva[i][4 * j + 3]};
+            f32x4{gv(dva[i][4 * j]), gv(dva[i][4 * j + 1]), gv(dva[i][4 * j + 2]), gv(dva[i][4 * j + 3])};
       }
   }
   return true;
