@@ -80,6 +80,27 @@ def _exact(q, k, v, do, scale, causal):
             (p @ np.abs(v), mds @ np.abs(k) * scale, t(mds) @ np.abs(q) * scale, t(p) @ np.abs(do)))
 
 
+# D 32: two groups in all three kernels, 64: in forward and dQ, 128: none
+@pytest.mark.parametrize("S,D,e", [(130, 32, 44), (300, 64, 44), (200, 128, 44), (300, 64, 33), (200, 128, 33),
+                                   (130, 32, 42)])
+def test_backward_of_large_inputs(S, D, e):
+    """Finite values from 2^e in V, dO and K, each in a head of its own next to a head without.  From 2^43 on the
+    work items that meet the K run on the float32 instructions, the others on the split, in one launch; below, and
+    with V and dO, all on the split (the sums stay finite)."""
+    import pallas_flexattn as pf
+    rng = np.random.default_rng(S)
+    q, k, v, do = (rng.standard_normal((1, 4, S, D)).astype(np.float32) for _ in range(4))
+    v[0, 0, S // 3] *= np.float32(2.0 ** e)
+    do[0, 1, S - 5, 3] = np.float32(2.0 ** e)
+    q[0, 2, :, 0] = 0.0                            # (scores as without)
+    k[0, 2, S // 2, 0] = np.float32(2.0 ** e)
+    got = _run(pf, q, k, v, do, pf.causal_mask)
+    want, mag = _exact(q, k, v, do, D ** -0.5, True)
+    for name, a, b, m in zip("o dq dk dv".split(), got, want, mag):
+        err = np.abs(a.astype(np.float64) - b)
+        assert np.all(np.isfinite(a)) and np.max(err / np.maximum(m, 1e-30)) < 1e-5, name
+
+
 @pytest.mark.parametrize("S,D", [(130, 32), (300, 64), (200, 128)])
 def test_backward_whose_scaled_sums_overflow(S, D):
     """Inputs of some 2^42 (below the line) in K, V and dO of one key and one query: dQ and dK pass 2^95, where sums of
