@@ -109,15 +109,6 @@ __device__ __forceinline__ float mod_score_t(const Problem& P, float raw, float 
   }
 }
 
-// Element (q, k) of a partial tile is kept: inside [lo, hi] (the interval
-// of keys the window / contiguous documents leave to query q, which also
-// bounds k below Skv) and, with a user mask, where the mask holds.
-template <class Mod>
-__device__ __forceinline__ bool mod_keep(const Problem& P, int b, int h, int q, int k, int lo, int hi) {
-  if constexpr (Mod::kMask) return k >= lo && k <= hi && Mod::mask(P, b, h, q, k);
-  else return k >= lo && k <= hi;
-}
-
 // Bits [max(lo, 0), min(hi, 31)] of a 32-position block (none when empty):
 // the positions of a partial tile that an interval mask keeps, one bit test per
 // element.  Compared element by element instead, the 16 to 32 conditions of a
