@@ -282,13 +282,15 @@ int fa_bwd_noalloc(const fa_params *p, const void *q, const void *k, const void 
  * compiling), FA_MODS_BUILTIN_SCORE only without FA_MODS_SCORE; a call whose
  * params set alibi_slopes or softcap needs a blob with FA_MODS_BUILTIN_SCORE
  * (FA_ERR_UNSUPPORTED otherwise).
+ * FA_MODS_GENERAL (when compiling): float32 kernels that use fewer registers and
+ * are slower, for a policy that the compiler fails on next to the usual ones.
  * fa_mods_compile (no GPU needed) returns a blob (malloc'd, release with
  * fa_mods_free_blob) holding the code object; fa_mods_load loads it on the
  * current GPU.  Kernel tiles are fixed: bf16 128 x 64 (forward, dQ) and
  * 128 keys x 64 queries (dK/dV); float32 128 x 32.  The bf16 kernels take
  * window / contiguous-document masks; document labels go into the user mask.
  */
-enum fa_mods_flags { FA_MODS_MASK = 1, FA_MODS_SCORE = 2, FA_MODS_BUILTIN_SCORE = 4 };
+enum fa_mods_flags { FA_MODS_MASK = 1, FA_MODS_SCORE = 2, FA_MODS_BUILTIN_SCORE = 4, FA_MODS_GENERAL = 8 };
 typedef struct fa_mods fa_mods;
 int fa_mods_compile(const char *policy_source, int dtype, int D, int flags, void **blob, size_t *blob_bytes,
                     char *log, size_t log_bytes);

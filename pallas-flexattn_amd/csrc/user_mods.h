@@ -46,13 +46,17 @@ struct BlobHeader {
 // policy's registers spilled on top the compiler (LLVM 22) crashed on two of
 // eight policies tried, in the pass that rewrites MFMA copies after spilling.
 // (Built-in masks: 680 us with the general kernel, 428 with the split one at
-// B2 H16 S2048 causal.)
-std::vector<std::string> mod_kernels(int dtype, int D, bool mods) {
+// B2 H16 S2048 causal.)  `general` (FA_MODS_GENERAL): all three, for policies
+// that are too much for the split forward or dQ.
+std::vector<std::string> mod_kernels(int dtype, int D, bool mods, bool general) {
   const std::string d = std::to_string(D), m = mods ? "true" : "false";
   if (dtype == FA_DTYPE_BF16)
     return {"fa::fwd_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>",
             "fa::dq_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>",
             "fa::dkdv_bf16_kernel<" + d + ", 64, 4, " + m + ", UserMod>"};
+  if (general)
+    return {"fa::fwd_kernel<float, " + d + ", 32, 4, " + m + ", UserMod>", "fa::dq_kernel<float, " + d + ", 32, 4, " + m + ", UserMod>",
+            "fa::dkdv_kernel<float, " + d + ", 32, 4, " + m + ", UserMod>"};
   return {"fa::fwd_f32_kernel<" + d + ", 4, " + m + ", UserMod>", "fa::dq_f32_kernel<" + d + ", 4, " + m + ", UserMod>",
           D == 128 ? "fa::dkdv_kernel<float, 128, 32, 4, " + m + ", UserMod>"
                    : "fa::dkdv_f32_kernel<" + d + ", 4, " + m + ", UserMod>"};
@@ -70,13 +74,16 @@ int compile_mods(const char* policy, int dtype, int D, int flags, std::vector<ch
   if (!policy || !blob) return FA_ERR_NULL;
   if (dtype != FA_DTYPE_BF16 && dtype != FA_DTYPE_F32) return FA_ERR_DTYPE;
   if (D != 32 && D != 64 && D != 128) return FA_ERR_UNSUPPORTED;
+  const bool general = (flags & FA_MODS_GENERAL) != 0;
+  if (general && dtype != FA_DTYPE_F32) return FA_ERR_UNSUPPORTED;
+  flags &= ~FA_MODS_GENERAL;  // (the blob's launches are the same)
   if (flags & ~(FA_MODS_MASK | FA_MODS_SCORE | FA_MODS_BUILTIN_SCORE)) return FA_ERR_UNSUPPORTED;
   // the built-in ALiBi / soft-cap epilogue runs only without a user score
   if ((flags & FA_MODS_SCORE) && (flags & FA_MODS_BUILTIN_SCORE)) return FA_ERR_UNSUPPORTED;
   // the kernels' score path runs when the user score or the built-in
   // ALiBi / soft-cap is present
   const bool mods = (flags & (FA_MODS_SCORE | FA_MODS_BUILTIN_SCORE)) != 0;
-  const std::vector<std::string> kernels = mod_kernels(dtype, D, mods);
+  const std::vector<std::string> kernels = mod_kernels(dtype, D, mods, general);
   std::string src = dtype == FA_DTYPE_BF16 ? "#include \"fwd_bf16.h\"\n#include \"bwd_bf16.h\"\n"
                                            : "#include \"f32_split.h\"\n";
   src += "\n";

@@ -81,7 +81,7 @@ EXPORTED = ("fa_fwd", "fa_fwd_fp8", "fa_fwd_fp8_q16", "fa_quantize_fp8", "fa_qua
             "fa_mods_compile", "fa_mods_free_blob", "fa_mods_load", "fa_mods_unload", "fa_mods_fwd", "fa_mods_bwd",
             "fa_mods_bwd_dkdv", "fa_mods_bwd_dq", "fa_mods_source_hash")
 
-MODS_MASK, MODS_SCORE, MODS_BUILTIN_SCORE = 1, 2, 4
+MODS_MASK, MODS_SCORE, MODS_BUILTIN_SCORE, MODS_GENERAL = 1, 2, 4, 8
 
 _lib = None
 _launch = None
@@ -236,7 +236,9 @@ sys.exit(0 if rc == 0 else 3)
 def compile_mods(source: str, dtype: int, head_dim: int, flags: int) -> bytes:
     """Compile a user-mods policy (C ABI fa_mods_compile, no GPU needed) in a
     child interpreter and return the code blob.  Raises FlexAttnError with
-    the compiler log."""
+    the compiler log.  Where the compiler itself dies on a float32 policy (it has,
+    with policies that need more registers than the kernels leave), the policy is
+    compiled into the general kernels (FA_MODS_GENERAL)."""
     import subprocess
     import sys
     import tempfile
@@ -245,8 +247,13 @@ def compile_mods(source: str, dtype: int, head_dim: int, flags: int) -> bytes:
     fd, out = tempfile.mkstemp(suffix=".blob")
     os.close(fd)
     try:
-        res = subprocess.run([sys.executable, "-c", _CHILD, LIB_PATH, str(dtype), str(head_dim), str(flags), out],
-                             input=source.encode(), capture_output=True, timeout=600)
+        def run(flags):
+            return subprocess.run([sys.executable, "-c", _CHILD, LIB_PATH, str(dtype), str(head_dim), str(flags), out],
+                                  input=source.encode(), capture_output=True, timeout=600)
+
+        res = run(flags)
+        if res.returncode < 0 and dtype == DTYPE_F32 and not flags & MODS_GENERAL:  # ended by a signal
+            res = run(flags | MODS_GENERAL)
         if res.returncode != 0:
             raise FlexAttnError(f"compiling the user mods failed (exit {res.returncode}):\n"
                                 f"{res.stderr.decode(errors='replace')[-8000:]}\n--- policy source ---\n{source}")

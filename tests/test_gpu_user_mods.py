@@ -231,3 +231,28 @@ def test_generated_functions_to_float32_rounding(name):
     _, lse = pf.flex_attention(q, k, torch.ones_like(k), score_mod=score, scale=1.0, return_lse=True)
     got = lse[0, 0].double().cpu().numpy()
     assert np.max(np.abs(got - want) / np.abs(want)) <= 8 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_general_float32_kernels_of_a_policy(D, monkeypatch, tmp_path):
+    """FA_MODS_GENERAL (what a policy gets that the compiler fails on next to the split kernels): forward and
+    backward against the oracle, ragged, grouped heads."""
+    import torch
+    from pallas_flexattn import _lib
+    pf = _pf()
+    compile_mods = _lib.compile_mods
+    monkeypatch.setattr(_lib, "compile_mods", lambda src, dt, d, flags: compile_mods(src, dt, d, flags | _lib.MODS_GENERAL))
+    monkeypatch.setenv("FLEXATTN_CACHE_DIR", str(tmp_path))  # (blobs of the usual kernels stay out)
+    S, Hq, Hkv = 200, 4, 2
+    q, k, v, do = inputs(40 + D, 1, Hq, Hkv, S, S, D, "fp32")
+    tq, tk, tv = (to_torch(x, "fp32").requires_grad_() for x in (q, k, v))
+    bm = pf.create_block_mask(lambda qi, kv: (qi >= kv) | (kv < 9), 1, Hq, S, S, 128)
+    o, lse = pf.flex_attention(tq, tk, tv, score_mod=lambda s, b, h, qi, kv: s - 0.03125 * s * s, block_mask=bm,
+                               enable_gqa=True, return_lse=True)
+    o.backward(to_torch(do, "fp32"))
+    assert b"9dq_kernelIfLi%d" % D in b"".join(p.read_bytes() for p in tmp_path.iterdir())
+    om = _dense_mask(lambda b, h, qi, kv: (qi >= kv) | (kv < 9), 1, Hq, S, S)
+    wo, wl, (wdq, wdk, wdv) = oracle_fwd_bwd(q, k, v, do, om,
+                                             score_fn=lambda s, b, h, qi, kv: (s - 0.03125 * s * s, 1.0 - 0.0625 * s))
+    for nm, got, want in (("O", o, wo), ("LSE", lse, wl), ("dQ", tq.grad, wdq), ("dK", tk.grad, wdk), ("dV", tv.grad, wdv)):
+        assert_close(f"general {nm}", to_np(got), want, FP32_TOL)

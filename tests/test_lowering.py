@@ -233,13 +233,20 @@ def test_derivative_of_integer_factors_is_a_float_product():
         assert "*dsds = (((float)(kv)) * ((float)(q)));" in body, body
 
 
-@pytest.mark.parametrize("name", ["tables", "functions"])
+@pytest.mark.parametrize("name", ["tables", "functions", "sine-and-tables"])
 def test_float32_policies_with_many_registers_compile(name):
-    """float32 at D = 128, where the kernels leave a policy the fewest registers: two table reads with a tanh, and
-    a sum of several functions (the compiler crashed on both next to a dK/dV kernel that fills the register file)."""
+    """float32 at D = 128, where the kernels leave a policy the fewest registers: table reads with a tanh, and a
+    sum of several functions (the compiler crashed on both next to a dK/dV kernel that fills the register file);
+    a sine with table reads crashes it next to dQ too and gets the general kernels."""
     from pallas_flexattn import _lib
-    t = torch.rand(2, 4, 64, 64)
+    t, near = torch.rand(2, 4, 64, 64), torch.rand(4, 128)
+
+    def sine(s, b, h, q, kv):
+        x = torch.clamp(s + 0.1 * torch.sin(s), min=-30.0, max=30.0) + t[b, h, q % 64, kv % 64]
+        return x + near[h, torch.clamp(q - kv, min=0, max=127)] + t[b, h, q % 64, kv % 64]
+
     mask, score = {
+        "sine-and-tables": (lambda b, h, q, kv: t[b, h, q % 64, kv % 64] > 0.3, sine),
         "tables": (lambda b, h, q, kv: t[b, h, q % 64, kv % 64] > 0.3,
                    lambda s, b, h, q, kv: s * t[b, h, kv % 64, q % 64] + t[b, h, q % 64, kv % 64] + 10 * torch.tanh(s / 10)),
         "functions": (lambda q, kv: ((q // 3) % 5 != (kv // 7) % 5) | (q == kv),
@@ -282,3 +289,16 @@ int main() {
     r = subprocess.run([str(tmp_path / "t")], capture_output=True, text=True)
     assert r.returncode == 0, r.returncode
     assert float(r.stdout) <= 2.5, r.stdout
+
+
+def test_general_float32_kernels_flag():
+    """FA_MODS_GENERAL: the general kernels by name, the same flags in the blob; float32 only; what compiling falls
+    back to when the compiler is ended by a signal."""
+    from pallas_flexattn import _lib
+    mods = L.UserMods(None, L.lower_score(lambda s, b, h, q, kv: s * 0.5))
+    f = mods.flags(False)
+    for flags, name in ((f, b"fwd_f32_kernel"), (f | _lib.MODS_GENERAL, b"10fwd_kernelIfLi64")):
+        blob = _lib.compile_mods(mods.source, _lib.DTYPE_F32, 64, flags)
+        assert int.from_bytes(blob[32:36], "little") == f and name in blob
+    with pytest.raises(_lib.FlexAttnError, match="exit 3"):
+        _lib.compile_mods(mods.source, _lib.DTYPE_BF16, 64, f | _lib.MODS_GENERAL)
