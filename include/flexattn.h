@@ -132,8 +132,8 @@ int fa_fwd(const fa_params *p, const void *q, const void *k, const void *v, void
  * query tile) walk is cut into n_splits key ranges computed by separate
  * workgroups, whose partial results (unnormalised O, running maximum and sum,
  * in the workspace) a second kernel merges into o and lse — the same outputs
- * as fa_fwd.  n_splits <= 0 picks two to five workgroups per CU with at least
- * four key tiles per split; at most 64.  Only the bf16 interval-mask kernel
+ * as fa_fwd.  n_splits <= 0 picks up to five workgroups per CU by the call's
+ * size, with at least four key tiles per split; at most 64.  Only the bf16 interval-mask kernel
  * splits; other problems run as fa_fwd (workspace unused).  No reference
  * counterpart (decode is on the reference's roadmap); workspace of
  * fa_fwd_splitkv_workspace_bytes(p, n_splits) bytes, 16-byte aligned. */

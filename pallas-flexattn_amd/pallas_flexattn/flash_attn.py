@@ -764,7 +764,7 @@ def flex_decode(query, key, value, score_mod: Optional[ScoreSpec] = None, block_
     """Forward-only FlexAttention for short query blocks against long key
     sequences (decoding).  The keys of each query tile are split into
     ``num_splits`` ranges computed by separate workgroups and merged by their
-    log-sum-exp (``None`` picks two to five workgroups per CU); with grouped-query
+    log-sum-exp (``None`` picks up to five workgroups per CU); with grouped-query
     attention the query heads sharing a kv head run as one tile, so each K / V
     tile is read once per group.  Same results as :func:`flex_attention`'s
     forward; no gradient.  The reference has no decode kernel (it is on its

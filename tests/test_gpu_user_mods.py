@@ -213,7 +213,7 @@ def test_builtin_score_params_need_a_blob_built_for_them():
 def test_generated_functions_to_float32_rounding(name):
     """With a single key the LSE is the score itself, so the generated tanh (polynomial below 0.8,
     exponential above) and the division by a constant are read off directly: every value within
-    8 * 2^-24 of float64 (4 of the function, 2 roundings of the log2 conversions, the input's scaling)."""
+    8 * 2^-24 of float64 (2.5 of the function, 2 roundings of the log2 conversions, the input's scaling)."""
     import torch
     pf = _pf()
     x = np.concatenate([np.geomspace(1e-6, 30.0, 2000), [0.49999997, 0.5, 0.50000006]]).astype(np.float32)
