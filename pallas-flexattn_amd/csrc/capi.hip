@@ -225,9 +225,9 @@ int fwd_launch(const fa_params* p, const fa_kv_cache* kv, const void* q, const v
   t.one_wave = one_wave && a.n_splits > 1;
   // rows of different lengths: an XCD that took whole batch rows (the L2 order)
   // would get more or less work than the others, so the heads go round the XCDs
-  // (128 heads of up to 7552 keys, five splits, L2 order / this: 78 / 62 us; 768
-  // of 1152 unsplit 65 / 60, 256 of 256 8.3 / 8.0).  Unsplit, with fewer items
-  // than units, it only costs (64 heads of 256 keys 9.6 / 10.0).
+  // (128 heads of up to 7552 keys, L2 order / this: in ten splits 78 / 62 us, in
+  // eight 64 / 63; 768 of 1152 unsplit 65 / 60, 256 of 256 8.3 / 8.0).  Unsplit,
+  // with fewer items than units, it only costs (64 heads of 256 keys 9.6 / 10.0).
   if (lens && one_wave && (a.n_splits > 1 || fwd_items(a.p, a.pack, t.bm) >= device_cus())) a.p.xcd_remap = 0;
   if (a.n_splits > 1) {
     if (!workspace || workspace_bytes < split_bytes(p, a.n_splits) || !aligned16({workspace}))

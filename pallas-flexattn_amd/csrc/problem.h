@@ -253,7 +253,7 @@ inline bool one_wave_fwd(const Problem& pr, int pack, int D, int cus) {
 // as many as give a CU (of cus) two workgroups, at least four key tiles per
 // split.  The one-wave workgroups of decode shapes:
 // * equal lengths, D = 64, three: a tile in flight is half as many bytes
-//   (128 heads of 30464 keys, 500 MB, with 1 / 2 / 3 / 4: 191 / 111 / 87 / 90 us);
+//   (64 kv heads of 30464 keys, 500 MB, with 1 / 2 / 3 / 4: 191 / 111 / 87 / 90 us);
 //   at D = 128 more than two only cost merging (B8 Hq32 Hkv8 Skv32768:
 //   184 / 191 / 205 us with 2 / 3 / 6);
 // * rows of different lengths (`lens`) balance over five (32 x 8 kv heads of up
@@ -263,7 +263,7 @@ inline bool one_wave_fwd(const Problem& pr, int pack, int D, int cus) {
 // * from two items per CU on, two splits are none: 512 items with 1 / 2 43 / 47
 //   us (D64, 1792 keys), lengths at D = 128 (896 keys) 31.5 / 35.1, 768 items with
 //   lengths at D = 64 (1152 keys) 31.3 / 33.8, but up to 1024 keys 20.8 / 19.4 (640);
-//   three only at D = 64 with lengths (512 items: 13 % faster than one).
+//   three only at D = 64 with lengths (512 items: a tenth faster than one).
 inline int choose_splits(const fa_params* p, const Tiles& t, const Problem& pr, int requested, int cus, bool lens) {
   if (p->dtype != FA_DTYPE_BF16 || !interval_masks(pr)) return 1;
   const int pack = choose_pack(p, t, pr);
